@@ -122,8 +122,10 @@ int mfr_event_elapsed_ms(mfr_event_t start, mfr_event_t end, float* ms);
  *
  * Each operand needs a unit stride in one of its two matrix dimensions (row-major or
  * transposed); C has column stride 1. c0 may equal c (in place). k == 0 gives the epilogue of
- * a zero product. The products are summed in fp32 on the fp32 matrix cores
- * (v_mfma_f32_32x32x2_f32), in a different order from the CPU's packed kernel.
+ * a zero product. The products are summed in fp32 on the matrix cores, in a different order from
+ * the CPU's packed kernel: up to a depth of 64 as fp32 products (v_mfma_f32_32x32x2_f32), above
+ * it as the six products of three-way bf16 parts that reach fp32 precision (their error against
+ * 64 bits is below the fp32 products'; what the parts cannot hold runs as fp32 products).
  *
  * Replaces: the Matmul kernel (src/backends/cpu/backend.cpp:131-164), the GemmBatched kernel
  * (backend.cpp:239-291), and the 4-dispatch composition of mensurflow::gemm
@@ -171,19 +173,19 @@ enum { MFR_GEMM_CAUSAL = 1 };
  * such operands in place, with 4-byte buffer loads that write LDS directly. */
 enum { MFR_STAGE_AUTO = 0, MFR_STAGE_NEVER = 1, MFR_STAGE_ALWAYS = 2 };
 
-/* Workgroup tile of mfr_sgemm (rows x cols x depth slice). AUTO picks one from the shape (with
- * the split count): a time model of the busiest CU's tiles (ceil(tiles / CUs) of them, each its
- * area x (depth + a fixed per-tile overhead) at the tile's measured rate, slower when a SIMD holds
- * fewer than 3 wavefronts), and the high-occupancy tiles for a depth <= 128. A fixed tile is what
+/* Workgroup tile of mfr_sgemm (rows x cols). AUTO picks one from the shape (with the split
+ * count): a time model of the busiest CU's tiles (ceil(tiles / CUs) of them, each its depth at
+ * the tile's measured rate plus a fixed time), and the 128x64 or 64x128 tile for a depth <= 64.
+ * A fixed tile is what
  * a tuner sets (the reference's TuningConfig,
  * src/core/dispatcher.hpp:145-149). Every tile gives the same results up to summation order. */
 enum {
     MFR_TILE_AUTO = 0,
-    MFR_TILE_256x256 = 1, /* 16 wavefronts of 64x64, 1 workgroup per CU */
-    MFR_TILE_128x128 = 2, /* 4 wavefronts of 64x64, 2 per CU */
-    MFR_TILE_128x64 = 3,  /* 4 wavefronts of 64x32, depth slice 16, up to 5 per CU */
-    MFR_TILE_64x128 = 4,  /* 4 wavefronts of 32x64, depth slice 16 */
-    MFR_TILE_64x64 = 5,   /* 4 wavefronts of 32x32, 4 per CU */
+    MFR_TILE_256x256 = 1, /* 8 wavefronts of 128x64, 1 workgroup per CU */
+    MFR_TILE_128x128 = 2, /* 8 wavefronts of 64x32, 1 per CU */
+    MFR_TILE_128x64 = 3,  /* 4 wavefronts of 64x32, 2 per CU (5 up to a depth of 64) */
+    MFR_TILE_64x128 = 4,  /* 4 wavefronts of 32x64, likewise */
+    MFR_TILE_64x64 = 5,   /* 4 wavefronts of 32x32, 3 per CU; or 8 of 64x64 sharing the depth */
     MFR_TILE_THIN = 6,    /* no MFMA: at most 8 output columns (or rows) as dot products */
     MFR_TILE_PANEL = 7,   /* k <= 64: 8 wavefronts keep 256 rows of A, stream B and C past them */
     MFR_TILE_COUNT = 8
@@ -209,7 +211,8 @@ enum {
  * multiple of 32 deep; fewer ranges than asked when the depth is short): each range's raw sums go
  * to the stream's workspace (splits * m * n * batch floats), and a second pass adds the ranges in
  * order and applies the epilogue with the same roundings. AUTO picks the tile and the count
- * together from a time model (no split when the output fills the device, ranges >= 256 deep,
+ * together from a time model (no split when the output fills the device, ranges >= 256 deep, 128 for
+ * the 64x64 tile,
  * partial sums <= 1 GiB) and falls back to no split when the workspace cannot be had; a fixed
  * count fails with MFR_E_RUNTIME then. Results are deterministic; the summation order, hence
  * the rounding, depends on the count. */

@@ -1,42 +1,32 @@
-// fp32 GEMM on the gfx950 fp32 matrix cores, with a fused epilogue (include/mfr_rocm.h,
-// mfr_sgemm):
+// fp32 GEMM on the gfx950 matrix cores, with a fused epilogue (include/mfr_rocm.h, mfr_sgemm):
 //
 //   C[b] = act( fl( fl( fl(alpha * op(A[b]) op(B[b])) + fl(beta * C0[b]) ) + bias ) )
 //
-// Design (a workgroup of 4 or 16 wavefronts of 64 lanes; five MFMA tile shapes and a thin path,
-// chosen per call with the split-K count and edge peeling, below):
-//   - The workgroup computes a BM x BN tile of C; its wavefronts form a WAVES_M x WAVES_N grid,
-//     each owning a (BM/WAVES_M) x (BN/WAVES_N) sub-tile held in 32x32 accumulator blocks of
-//     v_mfma_f32_32x32x2_f32 (16 fp32 accumulators per lane per block).
-//   - The depth is walked in slices of KT. Each slice of A (BM x KT) and B (KT x BN) is loaded
-//     from global memory into registers one slice ahead, then written to the other half of a
-//     double-buffered LDS tile, so one barrier per slice separates reads from writes.
-//   - Operand layout in LDS follows the operand's layout in memory, so the copy never
-//     transposes: a "K-major" operand (unit stride along the depth) is stored [rows][KT+4] and
-//     its MFMA fragments are single 16-byte LDS reads; an "M/N-major" operand (unit stride
-//     along its rows) is stored [KT][rows+8] and read as four 4-byte LDS reads. The pads keep
-//     both reads free of bank conflicts.
-//   - Depth permutation: within each group of 8 depth indices, lanes 0-31 of the wavefront feed
-//     depths 0-3 and lanes 32-63 depths 4-7 over four MFMA steps (step s uses depths s and
-//     4+s). A and B use the same permutation, so the sum is unchanged; it is what lets a
-//     K-major fragment be one 16-byte read.
+// Design (five workgroup tiles, a thin path and a panel path, chosen per call with the split-K
+// count and edge peeling, below):
+//   - Products deeper than 64 run on the bf16 matrix cores (split_kernel.hpp): each operand
+//     element is cut exactly into three bf16 parts, and six of the nine part products, summed in
+//     fp32, give the fp32 product with an error under a sequential fp32 sum's. Six products at 16
+//     times the fp32 rate: 4096^3 961 -> 555-607 us, the MLP 4093 x 1023 x 4099 282 -> 189 us,
+//     2048^3 137 -> 89 us. What the parts cannot hold (infinities, NaN, operands near either end
+//     of the exponent range) is found per tile and run again on the fp32 matrix cores.
+//   - Short depths run on the fp32 matrix cores (v_mfma_f32_32x32x2_f32; sgemm_kernel on the
+//     128x64 and 64x128 tiles, and the panel path): slices loaded a slice ahead into registers,
+//     then LDS, double-buffered, one barrier per slice.
+//   - Depth permutation (fp32 path): within each group of 8 depth indices, lanes 0-31 feed depths
+//     0-3 and lanes 32-63 depths 4-7 over four MFMA steps (step s uses depths s and 4+s), so a
+//     K-major fragment is one 16-byte read.
 //   - Tiles are handed out XCD-aware: hardware sends workgroup i to XCD i % 8, so consecutive
 //     logical tiles are remapped onto the same XCD (sharing its L2), and the logical order walks
 //     GROUP_M tile-rows at a time so concurrently running tiles share A and B panels.
-//   - Edges (M, N, K not multiples of the tile) are zero-filled on load and masked on store.
-//   - Operand staging: the 16-byte loads need an operand's lines (runs along its unit stride) to
-//     start 16-byte aligned and hold a multiple of 4 floats. An operand that is not laid out so
-//     (X[4093,1023] row-major) is copied first into the stream's workspace with its lines padded
-//     to a multiple of 4 by zeros (stage_kernel); vector loads that reach past the end of a line
-//     then read zeros of its own line, and the zeros add nothing to any sum. When a peeled strip
-//     of at most 8 columns covers every row of such an A, the strip's launch writes the copy as
-//     it reads A (strip_stage_kernel in thin_kernel.hpp), one launch instead of two.
-//   - Direct-to-LDS slices (sgemm_direct_kernel, the 256x256 tile with a 4-byte operand): each
-//     lane's buffer load writes its element into the LDS image itself, so 4-byte operands take
-//     no registers and need no staging copy; elements outside the matrix get an offset past the
-//     buffer's record limit and load as zeros. Its 16-byte form also replaces the register copy
-//     on aligned operands. Under it AUTO stages only K-major 4-byte operands (whose in-place
-//     runs of 32 floats touch twice the cache lines) and reads M/N-major ones in place.
+//   - Edges (M, N, K not multiples of the tile) are zero-filled or repeated on load and masked on
+//     store.
+//   - Operand staging: an operand whose lines (runs along its unit stride) do not start 16-byte
+//     aligned or hold a multiple of 4 floats (X[4093,1023] row-major) may be copied first into the
+//     stream's workspace with its lines padded to a multiple of 4 by zeros (stage_kernel); loads
+//     that reach past the end of a line then read zeros of its own line, and the zeros add nothing
+//     to any sum. When a peeled strip of at most 8 columns covers every row of such an A, the
+//     strip's launch writes the copy as it reads A (strip_stage_kernel in thin_kernel.hpp).
 //   - The epilogue applies the activation chosen once per workgroup, with copies for interior
 //     tiles and for C0, so each copy is straight-line code (gemm_kernel.hpp, write_tile); the
 //     tanh gelu's copies read its exp table from LDS and have no branch between elements.
@@ -45,6 +35,7 @@
 //     own; the thin path (thin_kernel.hpp) takes products with at most 8 output columns or rows.
 #include "gemm_kernel.hpp"
 #include "panel_kernel.hpp"
+#include "split.hpp"
 #include "thin_kernel.hpp"
 
 #include <cstring>
@@ -58,23 +49,29 @@ using namespace mfr::gemm;
 
 // ---- tile configurations ----------------------------------------------------------------------
 //
-// Five workgroup tiles (include/mfr_rocm.h, MFR_TILE_*). `tflops` is each tile's measured rate on
-// the 4096^3 NT problem (one MI355X) and `occupancy` its resident workgroups per CU (LDS and
-// registers); the automatic choice uses both.
+// Five workgroup tiles (include/mfr_rocm.h, MFR_TILE_*) with what a time model needs of each: the
+// workgroups a CU holds at once (LDS and registers), the time of one depth of a tile (us) with
+// 1, 2 or 3 of them resident, a tile's fixed time (first loads, exchange, write-out; shared by the
+// resident ones).
 struct TileInfo {
-    int bm, bn, occupancy, waves;
-    double tflops;
+    int bm, bn, occupancy;
+    double depth_us[3];
+    double fixed_us;
+    double full; // slower by this share on a chip full of them (power: a lower clock)
 };
 constexpr TileInfo kTiles[MFR_TILE_COUNT] = {
-    {0, 0, 0, 0, 0.0},         // AUTO
-    {256, 256, 1, 16, 135.3},  // 16 wavefronts of 64x64, depth slice 32
-    {128, 128, 2, 4, 127.3},   // 4 wavefronts of 64x64, depth slice 32
-    {128, 64, 5, 4, 114.9},    // 4 wavefronts of 64x32, depth slice 16
-    {64, 128, 5, 4, 116.0},    // 4 wavefronts of 32x64, depth slice 16
-    {64, 64, 4, 4, 111.4},     // 4 wavefronts of 32x32, depth slice 32
-    {0, 0, 0, 0, 0.0},         // THIN (no tile; priced by thin_us)
-    {0, 0, 0, 0, 0.0},         // PANEL (chosen by its own rule, panel_fits)
+    {0, 0, 0, {}, 0.0, 0.0},                             // AUTO
+    {256, 256, 1, {0.1051}, 5.0, 0.33},                    // 8 wavefronts of 128x64, slice 16
+    {128, 128, 1, {0.0348}, 2.5, 0.13},                    // 8 wavefronts of 64x32, slice 32
+    {128, 64, 2, {0.0318, 0.0256}, 2.2, 0.0},             // 4 wavefronts of 64x32, slice 32
+    {64, 128, 2, {0.0322, 0.0260}, 2.4, 0.0},             // 4 wavefronts of 32x64, slice 32
+    {64, 64, 3, {0.0171, 0.0153, 0.0146}, 1.8, 0.0},      // 4 wavefronts of 32x32, slice 32
+    {0, 0, 0, {}, 0.0, 0.0},                             // THIN (no tile; priced by thin_us)
+    {0, 0, 0, {}, 0.0, 0.0},                             // PANEL (chosen by its own rule, panel_fits)
 };
+constexpr double kRegsDepthUs = 0.0123; // the 64x64 tile's register form (regs_form)
+constexpr double kRegsFixedUs = 2.4;
+constexpr double kTileLaunchUs = 4.9;
 constexpr int kGroupM = 8;
 
 int64_t tile_count(int tile, int64_t m, int64_t n, int64_t batch) {
@@ -89,15 +86,12 @@ int64_t tile_count(int tile, int64_t m, int64_t n, int64_t batch) {
 // to the workspace; split_reduce_kernel adds them in order and applies the epilogue.
 
 constexpr int kMaxSplits = MFR_MAX_SPLITS;
-constexpr int64_t kMinAutoDepth = 256;           // AUTO never cuts a range shorter than this
 constexpr double kMaxPartialBytes = 1073741824.0; // AUTO keeps the partial sums under 1 GiB
-constexpr double kReduceBytesPerUs = 4.0e6;       // split_reduce_kernel's HBM rate (bytes/us)
-constexpr double kReduceLaunchUs = 4.0;           // its launch and ramp
-// A tile's fixed cost (first slice's load latency, writing the tile out), in depth-equivalents
-// of its MFMA work, shared among the workgroups a CU runs at once. Fit, with simd_efficiency, to
-// the measured times of every tile and split count on 14 shapes (64^2 x 65536 .. 8192^2 x 1024).
-constexpr double kTileOverheadDepth = 96.0;
+constexpr double kReduceBytesPerUs = 3.7e6;       // split_reduce_kernel's HBM rate (bytes/us)
+constexpr double kReduceLaunchUs = 2.4;           // its launch and ramp
 
+// AUTO never cuts a range shorter than this: two slices more than a tile's fixed time is worth.
+constexpr int64_t min_auto_depth(int tile) { return tile == MFR_TILE_64x64 ? 128 : 256; }
 // Depth of each range when `splits` are asked for: a multiple of 32, which every tile's depth
 // slice divides, so no range starts inside a slice.
 int64_t depth_per_split(int64_t k, int splits) {
@@ -107,37 +101,33 @@ int64_t depth_per_split(int64_t k, int splits) {
 
 int splits_for(int64_t k, int64_t per) { return static_cast<int>((k + per - 1) / per); }
 
-// Relative rate of a CU by how many wavefronts each SIMD holds: one alone hides no latency.
-double simd_efficiency(int64_t waves_per_simd) {
-    return waves_per_simd >= 3 ? 1.0 : waves_per_simd == 2 ? 0.9 : 0.85;
+// Whether an unsplit product of depth k runs `count` 64x64 tiles in the split kernel's register
+// form (sgemm_split_regs_kernel): every CU has at most one workgroup, and either more than half
+// of them have one or the depth is short; AUTO splits a longer depth over the idle CUs. 1024^3
+// 24.8 -> 20.7 us.
+bool regs_form(int64_t count, int64_t k, int cus) {
+    return count <= cus && (2 * count > cus || k <= 512);
 }
 
-// Modelled time (us) of tile t with `splits` depth ranges of `per` each: the busiest CU's share
-// of the tiles, each its depth plus the fixed overhead, at the tile's rate on 4096^3 (with the
-// overhead taken out), scaled by its wavefronts per SIMD relative to that measurement; plus the
-// reduce pass when split.
+// Modelled time (us) of tile t with `splits` depth ranges of `per` each: the launch, the busiest
+// CU's share of the tiles, and the reduce pass when split. The constants (kTiles, kRegs*,
+// kReduce*) were fit to 700 measured times of every tile with 1 to 64 ranges on 28 shapes from
+// 200^3 to 4096^3. On each shape the model's pick measures within 3 % of the
+// best point, 0.2 % on average.
 double modelled_us(int t, int64_t m, int64_t n, int64_t k, int64_t batch, int cus, int splits,
                    int64_t per, bool c0) {
     const TileInfo& info = kTiles[t];
     const int64_t count = tile_count(t, m, n, batch) * splits;
     const int64_t per_cu = (count + cus - 1) / cus;
-    const int64_t concurrent = per_cu < info.occupancy ? per_cu : info.occupancy;
-    // The 128x128 tile runs 8 wavefronts when no CU gets two (launch_layout). (The 64x64 tile
-    // then runs 16, four sets sharing each depth slice, but is priced as its 4-wavefront form:
-    // priced at 4 per SIMD, AUTO took it over split-K and the thin path where it is slower, e.g.
-    // 512^3 16.2 against 14.1 us, the MLP's 4093 x 3 strip 19.1 against 7.9 us.)
-    const int64_t waves = t == MFR_TILE_128x128 && count <= cus ? 8 : info.waves;
-    const int64_t reference_waves = (4096 / info.bm) * (4096 / info.bn) / 256;
-    const int64_t ref_concurrent =
-        reference_waves < info.occupancy ? reference_waves : info.occupancy;
-    const double efficiency = simd_efficiency(concurrent * waves / 4) /
-                              simd_efficiency(ref_concurrent * info.waves / 4);
+    const int64_t resident = per_cu < info.occupancy ? per_cu : info.occupancy;
+    const bool regs = t == MFR_TILE_64x64 && splits == 1 && regs_form(count, k, cus);
     const double depth = static_cast<double>(splits > 1 ? per : k);
-    const double overhead = kTileOverheadDepth / static_cast<double>(concurrent);
-    const double cu_flops_per_us = info.tflops * 1e6 / 256.0 *
-                                   (4096.0 + kTileOverheadDepth / ref_concurrent) / 4096.0;
-    double us = static_cast<double>(per_cu) * 2.0 * info.bm * info.bn * (depth + overhead) /
-                (cu_flops_per_us * efficiency);
+    const double tile_us = regs ? kRegsDepthUs * depth + kRegsFixedUs
+                                : info.depth_us[resident - 1] * depth +
+                                      info.fixed_us / static_cast<double>(resident);
+    const double fill = std::min(1.0, static_cast<double>(count) / cus);
+    double us = kTileLaunchUs + static_cast<double>(per_cu) * tile_us *
+                                    (1.0 + info.full * std::max(0.0, (fill - 0.56) / 0.44));
     if (splits > 1) {
         const double outputs = static_cast<double>(m) * n * batch;
         us += outputs * 4.0 * (2.0 * splits + (c0 ? 2.0 : 1.0)) / kReduceBytesPerUs +
@@ -173,7 +163,7 @@ int thin_b_layout(const GemmParams& p, const Plan& plan, int64_t m, int64_t n);
 // a cache-line access per value, so C > 1 takes 0.75 * C times as long (16384^2 x 1: 168 us;
 // 16384 x 4 x 4096: 125 us; 4096 x 8 x 1024: 22 us). Read in pieces, C = 2, 4 take 1.0 and 1.2
 // times as long (16384 x 2 x 4096: 43 us; 16384 x 4 x 4096: 51 us; 65536 x 4 x 512: 25 us);
-// C = 8 with B' staged in LDS 1.35 (16384 x 8 x 4096: 55.6 us; 65536 x 8 x 512: 31.6 us;
+// C = 8 with B' staged in LDS 1.27 (16384 x 8 x 4096: 55.6 us; 65536 x 8 x 512: 31.6 us;
 // 16384 x 8 x 1000: 15.3 us), 2.5 without (fewer than 16 rows). Slower in proportion with fewer
 // than 1024 wavefronts.
 double thin_us(int64_t m, int64_t n, int64_t k, int64_t batch, bool c0, bool ak, bool bk,
@@ -194,7 +184,7 @@ double thin_us(int64_t m, int64_t n, int64_t k, int64_t batch, bool c0, bool ak,
                           : !pieces      ? 0.75 * rounded
                           : rounded == 2.0 ? 1.0
                           : rounded == 4.0 ? 1.2
-                          : lds          ? 1.35
+                          : lds          ? 1.27
                                          : 2.5;
     return bytes / kThinBytesPerUs * factor * std::max(1.0, 1024.0 / waves) + kThinLaunchUs;
 }
@@ -207,8 +197,8 @@ struct Choice {
 };
 
 // The automatic tile and split count (either may be fixed by the caller: tile != AUTO, splits !=
-// 0). A short depth (K <= 128) is latency-bound per tile, so it takes the high-occupancy 128x64 /
-// 64x128 tiles (the one padding the output less). Otherwise the pair with the least modelled
+// 0). A short depth (up to the panel path's 64) takes the fp32 128x64 / 64x128 tiles (the one
+// padding the output less). Otherwise the pair with the least modelled
 // time. The thin path competes where it
 // can take the product (ak, bk: whether A and B are read along k) and no split is fixed.
 // big_ok: whether the 256x256 tile can read the operands (big_tile_ok).
@@ -240,7 +230,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int cus,
             best.per = k;
         }
     }
-    if (fixed_tile == MFR_TILE_AUTO && best.splits == 1 && k <= 128) {
+    if (fixed_tile == MFR_TILE_AUTO && best.splits == 1 && k <= kPanelMaxDepth) {
         const int64_t a = tile_count(MFR_TILE_128x64, m, n, batch) * 128 * 64;
         const int64_t b = tile_count(MFR_TILE_64x128, m, n, batch) * 64 * 128;
         best.tile = b < a ? MFR_TILE_64x128 : MFR_TILE_128x64;
@@ -271,7 +261,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int cus,
                 }
                 prev = splits;
                 if (splits > 1 &&
-                    (per < kMinAutoDepth ||
+                    (per < min_auto_depth(t) ||
                      4.0 * splits * static_cast<double>(m) * n * batch > kMaxPartialBytes)) {
                     break;
                 }
@@ -340,104 +330,55 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmParams p) {
     }
 }
 
-template <int BM, int BN, int KT, int WAVES_M, int WAVES_N, bool AK, bool BK, int WAVES_K = 1>
+template <int BM, int BN, int KT, int WAVES_M, int WAVES_N, bool AK, bool BK>
 void launch_vec(const GemmParams& p, int va, int vb, unsigned blocks, hipStream_t stream) {
-    constexpr int threads = WAVES_M * WAVES_N * WAVES_K * 64;
+    constexpr int threads = WAVES_M * WAVES_N * 64;
     if (va == 4 && vb == 4) {
-        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 4, 4, WAVES_K>
-            <<<blocks, threads, 0, stream>>>(p);
+        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 4, 4><<<blocks, threads, 0, stream>>>(p);
     } else if (va == 4) {
-        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 4, 1, WAVES_K>
-            <<<blocks, threads, 0, stream>>>(p);
+        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 4, 1><<<blocks, threads, 0, stream>>>(p);
     } else if (vb == 4) {
-        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 1, 4, WAVES_K>
-            <<<blocks, threads, 0, stream>>>(p);
+        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 1, 4><<<blocks, threads, 0, stream>>>(p);
     } else {
-        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 1, 1, WAVES_K>
-            <<<blocks, threads, 0, stream>>>(p);
+        sgemm_kernel<BM, BN, KT, WAVES_M, WAVES_N, AK, BK, 1, 1><<<blocks, threads, 0, stream>>>(p);
     }
 }
 
-// one_per_cu: no CU gets more than one workgroup. The 128x128 tile then runs 8 wavefronts of
-// 64x32 (2 per SIMD) instead of 4 of 64x64: 2048^3 145 against 155 us. With two workgroups per
-// CU the 4 wavefronts are faster (4096^3 1075 against 1105 us). Unsplit, the 128x128 tile
-// then runs 16 wavefronts in two sets and the 64x64 tile 16 in four, the sets sharing each
-// depth slice.
-// Whether the direct-to-LDS loaders' 32-bit byte offsets hold a bm x kt slice of A and a bn x kt
-// slice of B: every element of a slice lies below 2^30 bytes from its first (A(m, k) at
-// a + m a_rs + k a_cs, B(k, n) at b + k b_rs + n b_cs; a K-major operand's lines are its rows, an
-// M/N-major one's its depths, so deep slices of an M/N-major operand span kt - 1 line strides).
 template <bool AK, bool BK>
-bool direct_slices_fit(const GemmParams& p, int64_t bm, int64_t bn, int64_t kt) {
-    const auto extent = [kt](bool kmaj, int64_t rows, int64_t line) {
-        return kmaj ? (rows - 1) * line + kt : (kt - 1) * line + rows;
-    };
-    const int64_t a_line = AK ? p.a_rs : p.a_cs;
-    const int64_t b_line = BK ? p.b_cs : p.b_rs;
-    constexpr int64_t kLimit = int64_t{1} << 28; // floats
-    return a_line >= 0 && b_line >= 0 && a_line < kLimit && b_line < kLimit &&
-           extent(AK, bm, a_line) < kLimit && extent(BK, bn, b_line) < kLimit;
+void launch_layout(int tile, const GemmParams& p, int va, int vb, unsigned blocks,
+                   hipStream_t stream) {
+    if (tile == MFR_TILE_128x64) {
+        launch_vec<128, 64, 16, 2, 2, AK, BK>(p, va, vb, blocks, stream);
+    } else {
+        launch_vec<64, 128, 16, 2, 2, AK, BK>(p, va, vb, blocks, stream);
+    }
 }
 
-template <bool AK, bool BK>
-void launch_layout(int tile, const GemmParams& p, int va, int vb, unsigned blocks, bool one_per_cu,
-                   hipStream_t stream) {
-    // With one workgroup per CU, no split and 16-byte operands, the 64x64 and 128x128 tiles run
-    // the direct-to-LDS kernel (one accumulation chain, the tile kernels' depth order) in place of
-    // the wavefront sets, on slices as deep as the CU's LDS allows (128 and 64: 138-148 KiB), so
-    // each slice's MFMA work covers the next slice's load: 1024^3 28.9-29.5 -> 25.1-25.4 us,
-    // 2048^3 146.2-152.2 -> 135.7-138.3 us across the four layouts.
-    const auto direct_mid = [&](int64_t bm, int64_t bn, int64_t kt) {
-        return one_per_cu && p.splits == 1 && va == 4 && vb == 4 &&
-               direct_slices_fit<AK, BK>(p, bm, bn, kt);
-    };
+// Whether a tile runs the split kernel (bf16 matrix cores, split_kernel.hpp) on a product of depth
+// k. The 128x64 and 64x128 tiles, which AUTO takes for short depths, keep the fp32 matrix cores up
+// to the panel path's 64: there the products are one or two slices and bound by latency and the
+// output, and the two paths give the same bits.
+bool split_takes(int tile, int64_t k) {
+    return (tile != MFR_TILE_128x64 && tile != MFR_TILE_64x128) || k > kPanelMaxDepth;
+}
+
+// `blocks` workgroups of `tile` on the split kernel.
+void launch_split(int tile, const GemmParams& q, bool ak, bool bk, unsigned blocks, int cus,
+                  hipStream_t stream) {
+    constexpr int64_t kFarLines = int64_t{1} << 26; // the register form's 32-bit offsets
+    const bool near = (ak || q.a_cs < kFarLines) && (bk || q.b_rs < kFarLines);
     switch (tile) {
-    case MFR_TILE_256x256:
-        // The direct-to-LDS form for every load width: with 16-byte operands it also beats the
-        // register copy (4096^3 NT 1039 against 1075 us, 4096x4096x1024 286 against 300 us, the
-        // same bits).
-        if (va == 4 && vb == 4) {
-            sgemm_direct_kernel<256, 256, 32, 4, 4, AK, BK, 4, 4><<<blocks, 1024, 0, stream>>>(p);
-        } else if (va == 4) {
-            sgemm_direct_kernel<256, 256, 32, 4, 4, AK, BK, 4, 1><<<blocks, 1024, 0, stream>>>(p);
-        } else if (vb == 4) {
-            sgemm_direct_kernel<256, 256, 32, 4, 4, AK, BK, 1, 4><<<blocks, 1024, 0, stream>>>(p);
-        } else {
-            sgemm_direct_kernel<256, 256, 32, 4, 4, AK, BK, 1, 1><<<blocks, 1024, 0, stream>>>(p);
-        }
-        break;
-    case MFR_TILE_128x64:
-        launch_vec<128, 64, 16, 2, 2, AK, BK>(p, va, vb, blocks, stream);
-        break;
-    case MFR_TILE_64x128:
-        launch_vec<64, 128, 16, 2, 2, AK, BK>(p, va, vb, blocks, stream);
-        break;
+    case MFR_TILE_256x256: launch_split_256x256(q, ak, bk, blocks, stream); break;
+    case MFR_TILE_128x64: launch_split_128x64(q, ak, bk, blocks, stream); break;
+    case MFR_TILE_64x128: launch_split_64x128(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x64:
-        if (direct_mid(64, 64, 128)) {
-            sgemm_direct_kernel<64, 64, 128, 2, 2, AK, BK, 4, 4><<<blocks, 256, 0, stream>>>(p);
-        } else if (one_per_cu && p.splits == 1) {
-            // 16 wavefronts: four sets of 2x2 share each 64-deep slice (4 per SIMD). 1024^3:
-            // 31.0 -> 27.7 us; 16384 x 4 x 4096: 113.7 -> 94.2 us. Split depth ranges are
-            // short and keep the 4-wavefront form (512^3 in two: 14.5 against 14.1 us).
-            launch_vec<64, 64, 64, 2, 2, AK, BK, 4>(p, va, vb, blocks, stream);
+        if (q.splits == 1 && regs_form(blocks, q.k, cus) && near) {
+            launch_split_regs_64x64(q, ak, bk, blocks, stream);
         } else {
-            launch_vec<64, 64, 32, 2, 2, AK, BK>(p, va, vb, blocks, stream);
+            launch_split_64x64(q, ak, bk, blocks, stream);
         }
         break;
-    default:
-        if (direct_mid(128, 128, 64)) {
-            sgemm_direct_kernel<128, 128, 64, 4, 4, AK, BK, 4, 4><<<blocks, 1024, 0, stream>>>(p);
-        } else if (one_per_cu && p.splits == 1) {
-            // 16 wavefronts: two sets of 2x4 share each 64-deep slice (4 per SIMD). 2048^3:
-            // 150.2 -> 145.6 us; 2048 x 2048 x 8192: 583.9 -> 560.9 us (32-deep slices: 149.3
-            // and 574.1 us).
-            launch_vec<128, 128, 64, 2, 4, AK, BK, 2>(p, va, vb, blocks, stream);
-        } else if (one_per_cu) {
-            launch_vec<128, 128, 32, 2, 4, AK, BK>(p, va, vb, blocks, stream);
-        } else {
-            launch_vec<128, 128, 32, 2, 2, AK, BK>(p, va, vb, blocks, stream);
-        }
-        break;
+    default: launch_split_128x128(q, ak, bk, blocks, stream); break;
     }
 }
 
@@ -625,15 +566,19 @@ void single_region(Plan& plan, const Choice& choice) {
 // whole extra wave of tiles for a sliver of work. In AUTO, such a remainder (at most a quarter of
 // the tile) may be peeled off: the main rectangle runs on the big tile, and each edge strip runs
 // as a launch of its own, with its own tile and split count. The peeled plan is kept when the
-// model prices it (plus kLaunchUs per extra launch) at least 5% below the best single launch.
+// model prices it (plus kLaunchUs per extra launch) at least 5% below the best single launch, or
+// no more than 5% above it for a sliver off a large product.
 constexpr double kLaunchUs = 5.0;
 constexpr double kPeelMargin = 0.95;
+// A sliver of at most 8 rows or columns is peeled off unless that is priced this much higher: the
+// model is no nearer than that (3 x 2049 x 2047 x 2048: 274 us whole, 284 in two).
+constexpr double kSliverMargin = 1.05;
 
 bool big_tile_ok(const Plan& plan);
 
 void consider_peeling(Plan& plan, int64_t batch, int cus, double single_us) {
     const GemmParams& p = plan.p;
-    double best_us = single_us * kPeelMargin;
+    double best_us = single_us;
     for (int t = 1; t < MFR_TILE_THIN; ++t) {
         const int64_t bm = kTiles[t].bm, bn = kTiles[t].bn;
         const int64_t rem_m = p.m % bm, rem_n = p.n % bn;
@@ -667,6 +612,9 @@ void consider_peeling(Plan& plan, int64_t batch, int cus, double single_us) {
         if (peel_m && peel_n) {
             strip(main_m, main_n, rem_m, rem_n);
         }
+        const bool sliver = (!peel_m || rem_m <= 8) && (!peel_n || rem_n <= 8) &&
+                            2.0 * p.m * p.n * p.k * batch >= 17179869184.0;
+        us /= sliver ? kSliverMargin : kPeelMargin;
         if (us < best_us) {
             best_us = us;
             plan.region_count = count;
@@ -1062,14 +1010,6 @@ bool streamed_output(const GemmParams& q) {
     return true;
 }
 
-// Whether the 128x64 tile runs as sgemm_pair_kernel on q: A read along k and B along n, both by
-// 16-byte loads, one tile of columns (n <= 64), and each slice's byte offsets below 2^30 (the
-// direct-to-LDS loaders' 32-bit offsets, as big_tile_ok).
-bool pair_fits(const Plan& plan, const GemmParams& q, int va, int vb) {
-    return plan.ak && !plan.bk && va == 4 && vb == 4 && q.n <= 64 &&
-           127.0 * q.a_rs + 32.0 < 268435456.0 && 31.0 * q.b_rs + 64.0 < 268435456.0;
-}
-
 // Launches the kernel (and the reduce, when split) for region r of the product p describes.
 void launch_region(const Plan& plan, const GemmParams& p, const Region& r, int va, int vb,
                    float* partial, int cus, hipStream_t stream, float* stage = nullptr,
@@ -1107,17 +1047,16 @@ void launch_region(const Plan& plan, const GemmParams& p, const Region& r, int v
     q.partial = r.splits > 1 ? partial : nullptr;
     q.stream_c = q.partial == nullptr && streamed_output(q) ? 1 : 0;
     const unsigned grid = static_cast<unsigned>(blocks);
-    const bool one_per_cu = blocks <= cus;
-    if (tile == MFR_TILE_128x64 && pair_fits(plan, q, va, vb)) {
-        sgemm_pair_kernel<32><<<grid, 256, 0, stream>>>(q);
+    if (split_takes(tile, q.k)) {
+        launch_split(tile, q, plan.ak, plan.bk, grid, cus, stream);
     } else if (plan.ak && plan.bk) {
-        launch_layout<true, true>(tile, q, va, vb, grid, one_per_cu, stream);
+        launch_layout<true, true>(tile, q, va, vb, grid, stream);
     } else if (plan.ak) {
-        launch_layout<true, false>(tile, q, va, vb, grid, one_per_cu, stream);
+        launch_layout<true, false>(tile, q, va, vb, grid, stream);
     } else if (plan.bk) {
-        launch_layout<false, true>(tile, q, va, vb, grid, one_per_cu, stream);
+        launch_layout<false, true>(tile, q, va, vb, grid, stream);
     } else {
-        launch_layout<false, false>(tile, q, va, vb, grid, one_per_cu, stream);
+        launch_layout<false, false>(tile, q, va, vb, grid, stream);
     }
     mfr::check_launch("sgemm_kernel");
     if (q.partial != nullptr) {

@@ -1,0 +1,18 @@
+// Launches of the split tile kernel (split_kernel.hpp), one translation unit per tile shape.
+#pragma once
+
+#include "gemm_kernel.hpp"
+
+namespace mfr::gemm {
+
+// p's tile fields are filled for the tile; ak, bk: A and B are read along k.
+void launch_split_256x256(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
+void launch_split_128x128(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
+void launch_split_128x64(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
+void launch_split_64x128(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
+// No LDS in the depth loop; M/N-major lines less than 2^26 floats apart.
+void launch_split_regs_64x64(const GemmParams& p, bool ak, bool bk, unsigned blocks,
+                             hipStream_t s);
+void launch_split_64x64(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
+
+} // namespace mfr::gemm

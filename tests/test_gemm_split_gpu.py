@@ -1,0 +1,124 @@
+"""The GEMM tiles on the bf16 matrix cores (three bf16 parts per operand element) where the parts
+could miss the fp32 product: non-finite and huge operands, tiny ones, sums that are zero or
+underflow, at tile edges and remainders of the 16- and 32-deep slices. Against float64 products
+rounded to float32, within the summation bound k * 2^-24 of sum |a b| (plus the float32 product's
+own underflow, 2^-149 per term)."""
+import numpy as np
+import pytest
+
+import mensurflow_amd as mf
+
+pytestmark = pytest.mark.gpu
+
+TILES = [mf.abi.TILE_256x256, mf.abi.TILE_128x128, mf.abi.TILE_128x64, mf.abi.TILE_64x128,
+         mf.abi.TILE_64x64]
+
+
+def check(stream, a, b, tile, trans_a=False, trans_b=False, splits=1):
+    """One product against its float64 value; returns the result."""
+    m, k = a.shape
+    n = b.shape[1]
+    a_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(a.T if trans_a else a), stream)
+    b_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(b.T if trans_b else b), stream)
+    got = mf.gemm(a_d, b_d, trans_a=trans_a, trans_b=trans_b, tile=tile, splits=splits,
+                  stage=mf.abi.STAGE_NEVER).numpy()
+    with np.errstate(all="ignore"):
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        want = (a64 @ b64).astype(np.float32)
+        scale = np.abs(a64) @ np.abs(b64)
+    what = f"tile {tile} {m}x{n}x{k} ta {trans_a} tb {trans_b}"
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)), what
+    assert np.array_equal(got[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)]), what
+    bound = scale * k * 2.0**-24 + k * 2.0**-149
+    err = np.abs(got[finite].astype(np.float64) - want[finite].astype(np.float64))
+    assert np.all(err <= bound[finite]), (what, float(np.max(err / bound[finite])))
+    return got
+
+
+def normal(shape, seed, scale=1.0):
+    return (np.random.default_rng(seed).standard_normal(shape) * scale).astype(np.float32)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 65), (37, 70, 80), (130, 257, 95), (64, 64, 1000),
+                                   (300, 260, 129), (1000, 1000, 97)])
+def test_normal_operands(stream, tile, m, n, k):
+    for ta in (False, True):
+        for tb in (False, True):
+            check(stream, normal((m, k), 1), normal((k, n), 2), tile, ta, tb)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("case", ["inf", "inf times zero", "nan", "huge", "overflow", "tiny",
+                                  "tiny and large", "tiny product", "denormal", "zero rows",
+                                  "zeros", "few tiny", "identity"])
+def test_extreme_operands(stream, tile, case):
+    # 16 x 16 tiles of 64x64: the register form; fewer workgroups than half the CUs: the other.
+    for m, n, k in ((1000, 1000, 71), (150, 90, 200)):
+        a, b = normal((m, k), 3), normal((k, n), 4)
+        if case == "inf":
+            a[5, 3], a[m - 1, k - 1], b[7, 11] = np.inf, -np.inf, np.inf
+        elif case == "inf times zero":
+            a[5, 3], b[3, 8], a[6, 3] = np.inf, 0.0, 1.0
+        elif case == "nan":
+            a[m - 1, 0], b[k - 1, n - 1] = np.nan, np.nan
+        elif case == "huge":  # above the largest bf16, the products finite
+            a[2, 1], b[1, :] = 3.4e38, np.float32(1e-3)
+            a[9, 4], b[4, :] = -3.4e38, np.float32(2.0**-40)
+        elif case == "overflow":
+            a[2, :], b[:, 9] = 1e30, 1e30
+        elif case == "tiny":
+            a = normal((m, k), 3, 1e-36)
+        elif case == "tiny and large":
+            a, b = normal((m, k), 3, 1e-38), normal((k, n), 4, 1e30)
+        elif case == "tiny product":
+            a, b = normal((m, k), 3, 1e-20), normal((k, n), 4, 1e-19)
+        elif case == "denormal":
+            a = normal((m, k), 3, 1e-41)
+            b = normal((k, n), 4, 1e20)
+        elif case == "zero rows":
+            a[m // 3: m // 2], b[:, n // 2:] = 0.0, 0.0
+            a[m // 3, 2] = 1e-40
+        elif case == "zeros":
+            a[:] = 0.0
+        elif case == "few tiny":  # sums clear of what the tiny elements can lose
+            a[:, 1::3] = normal((m, k), 5, 1e-39)[:, 1::3]
+        elif case == "identity":  # every element comes back exactly
+            b = np.zeros((k, n), np.float32)
+            b[np.arange(min(k, n)), np.arange(min(k, n))] = 1.0
+        got = check(stream, a, b, tile)
+        if case == "identity":
+            q = min(k, n)
+            assert np.array_equal(got[:, :q], a[:, :q])
+
+
+def test_one_zero_sum(stream):
+    """A sum that is exactly zero among ordinary ones (its row and column are read again)."""
+    for tile in TILES:
+        a, b = normal((300, 128), 6), normal((128, 300), 7)
+        a[17, 64:] = -a[17, :64]
+        b[64:, 31] = b[:64, 31]
+        got = check(stream, a, b, tile)
+        assert abs(got[17, 31]) <= 128 * 2.0**-24 * np.abs(a[17]) @ np.abs(b[:, 31])
+
+
+@pytest.mark.parametrize("splits", [2, 5])
+def test_extremes_in_depth_ranges(stream, splits):
+    a, b = normal((200, 700), 8), normal((700, 130), 9)
+    a[3, 10], b[650, 100], a[50] = np.inf, np.nan, 1e-41
+    check(stream, a, b, mf.abi.TILE_64x64, splits=splits)
+
+
+def test_no_larger_error_than_fp32_chains(stream):
+    """The 2-norm error on uniform and normal operands stays under a sequential fp32 sum's
+    (sqrt(k) / 4 roundings of 2^-24 at the sum's size), whatever the tile."""
+    for k in (128, 1024, 4096):
+        a = np.random.default_rng(k).uniform(-1, 1, (256, k)).astype(np.float32)
+        b = np.random.default_rng(k + 1).uniform(-1, 1, (k, 256)).astype(np.float32)
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        for tile in TILES:
+            got = mf.gemm(mf.DeviceArray.from_numpy(a, stream),
+                          mf.DeviceArray.from_numpy(b, stream), tile=tile, splits=1).numpy()
+            rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+            assert rel <= np.sqrt(k) * 2.0**-24 * 0.3, (k, tile, rel)
