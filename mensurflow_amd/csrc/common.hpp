@@ -167,6 +167,25 @@ __device__ inline float4 load_streaming(const float* p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
+// 16-byte loads of 4 floats at any 4-byte aligned address, which the memory unit takes at the
+// rate of aligned ones but for the cache lines they straddle.
+typedef native_float4 loose_float4 __attribute__((aligned(4)));
+
+__device__ inline float4 load_loose(const float* p) {
+    const native_float4 v = *reinterpret_cast<const loose_float4*>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+__device__ inline float4 load_streaming_loose(const float* p) {
+    const native_float4 v = __builtin_nontemporal_load(reinterpret_cast<const loose_float4*>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+__device__ inline void store_loose(float* p, float4 v) {
+    const native_float4 n = {v.x, v.y, v.z, v.w};
+    *reinterpret_cast<loose_float4*>(p) = n;
+}
+
 __device__ inline double wave_sum(double v) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {

@@ -7,20 +7,28 @@
 // fused multiply-add in double rounds exactly like the reference's multiply-then-add; only the
 // order of the additions differs, and it is fixed, so every call gives the same bits.
 //
-// N form (y has `rows` entries): one wavefront owns kRowsPerWave (8) rows and walks them with
-// 16-byte loads, kUnrollN loads per row in flight per lane; each x chunk is read once for all 8
-// rows. The partial sums are reduced across the wavefront with shuffles. Every byte of A is read
-// once, coalesced. Workgroups of 2 wavefronts stream 16 consecutive rows; at 16384 rows that is
-// 1024 workgroups (4 per CU), one round of the chip. Measured against 4 rows per wavefront in
-// workgroups of 4: 6.89 vs 6.52 TB/s, the read rate of a plain contiguous stream (6.92 TB/s).
+// N form (y has `rows` entries), many aligned rows: one wavefront owns kRowsPerWave (8) rows and
+// walks them with 16-byte loads, kUnrollN loads per row in flight per lane; each x chunk is read
+// once for all 8 rows. The partial sums are reduced across the wavefront with shuffles. Every byte
+// of A is read once, coalesced. Workgroups of 2 wavefronts stream 16 consecutive rows; at 16384
+// rows that is 1024 workgroups (4 per CU), one round of the chip. Measured against 4 rows per
+// wavefront in workgroups of 4: 6.89 vs 6.52 TB/s, the read rate of a plain contiguous stream
+// (6.92 TB/s).
+//
+// N form, fewer rows or unaligned ones: a workgroup's wavefronts share the columns of 4 rows, or
+// of one (gemv_n_shared_kernel). One wavefront per 8 rows left most of the chip idle, and read
+// unaligned rows one float per lane: 64 x 16384 23.5 -> 4.1 us, 500 x 9001 25.6 -> 5.6, 4096^2
+// 23.2 -> 13.1, 4095 x 4097 25.3 -> 12.8, 16383 x 16381 201 -> 173.
 //
 // T form (y has `cols` entries): a workgroup of one wavefront owns a strip of 256 columns
 // (64 lanes x 4) and a chunk of rows, walks the rows in order with kUnrollT rows in flight, and
 // each lane keeps 4 column sums. The chunk's partial sums go to the stream's workspace
-// ([chunks][cols] doubles) and a second kernel adds the chunks in order. A is again read once,
-// coalesced along the rows. At 16384^2: 64 strips x 32 chunks = 2048 wavefronts. Measured
-// against four wavefronts splitting each chunk's rows (exchanging sums in LDS) with 8 rows in
-// flight: 6.96 vs 6.44 TB/s.
+// ([chunks][cols] doubles) and a second kernel adds the chunks in a fixed order. A is again read
+// once, coalesced along the rows, at any alignment. At 16384^2: 64 strips x 32 chunks = 2048
+// wavefronts. Measured against four wavefronts splitting each chunk's rows (exchanging sums in
+// LDS) with 8 rows in flight: 6.96 vs 6.44 TB/s. Chunks of 16 rows at the least and a second
+// kernel whose loads overlap: 4093 x 1023 86.6 -> 10.5 us, 8192 x 1024 32.9 -> 14.6, 16384 x 256
+// 67.5 -> 17.3, 16383 x 16381 908 -> 172 (one float per lane before).
 #include "common.hpp"
 
 namespace {
@@ -41,8 +49,8 @@ __device__ inline float finish(double sum, float alpha, float beta, const float*
 // Per-lane sums of rows row0 .. row0 + kRowsPerWave - 1 of A times x. FULL: all kRowsPerWave
 // rows exist, so they are lda apart from row0 and the compiler walks them from one base (that
 // schedule streams faster); otherwise rows past the end repeat the last valid row, and their sums
-// are never stored. VEC4: rows start 16-byte aligned and cols % 4 == 0 (checked on the host).
-template <bool VEC4, bool FULL>
+// are never stored. Rows start 16-byte aligned and cols % 4 == 0 (checked on the host).
+template <bool FULL>
 __device__ inline void gemv_n_rows(const float* __restrict__ a, int64_t lda,
                                    const float* __restrict__ x, int64_t cols, int64_t row0,
                                    int nrows, int lane, double (&sum)[kRowsPerWave]) {
@@ -52,7 +60,7 @@ __device__ inline void gemv_n_rows(const float* __restrict__ a, int64_t lda,
         sum[r] = 0.0;
         arow[r] = a + (row0 + (FULL || r < nrows ? r : nrows - 1)) * lda;
     }
-    if constexpr (VEC4) {
+    {
         const int64_t quads = cols / 4;                              // float4 per row
         const int64_t step = static_cast<int64_t>(kWave) * kUnrollN; // quads per iteration
         const int64_t main_quads = quads / step * step;
@@ -91,18 +99,9 @@ __device__ inline void gemv_n_rows(const float* __restrict__ a, int64_t lda,
                 sum[r] = fma(static_cast<double>(av.w), static_cast<double>(xv.w), sum[r]);
             }
         }
-    } else {
-        for (int64_t j = lane; j < cols; j += kWave) {
-            const double xj = static_cast<double>(x[j]);
-#pragma unroll
-            for (int r = 0; r < kRowsPerWave; ++r) {
-                sum[r] = fma(static_cast<double>(arow[r][j]), xj, sum[r]);
-            }
-        }
     }
 }
 
-template <bool VEC4>
 __global__ __launch_bounds__(kWave* kWavesPerBlockN) void gemv_n_kernel(
     const float* __restrict__ a, int64_t lda, const float* __restrict__ x, int64_t rows,
     int64_t cols, float alpha, float beta, const float* __restrict__ y0, float* __restrict__ y) {
@@ -115,9 +114,9 @@ __global__ __launch_bounds__(kWave* kWavesPerBlockN) void gemv_n_kernel(
     const int nrows = rows - row0 < kRowsPerWave ? static_cast<int>(rows - row0) : kRowsPerWave;
     double sum[kRowsPerWave];
     if (nrows == kRowsPerWave) {
-        gemv_n_rows<VEC4, true>(a, lda, x, cols, row0, nrows, lane, sum);
+        gemv_n_rows<true>(a, lda, x, cols, row0, nrows, lane, sum);
     } else {
-        gemv_n_rows<VEC4, false>(a, lda, x, cols, row0, nrows, lane, sum);
+        gemv_n_rows<false>(a, lda, x, cols, row0, nrows, lane, sum);
     }
 #pragma unroll
     for (int r = 0; r < kRowsPerWave; ++r) {
@@ -130,13 +129,94 @@ __global__ __launch_bounds__(kWave* kWavesPerBlockN) void gemv_n_kernel(
     }
 }
 
+// N form for rows that the streaming form cannot read or fill the chip with: a workgroup of WAVES
+// wavefronts owns R rows, its wavefronts share the columns (interleaved blocks of 256, 16-byte
+// loads, 4-byte aligned suffices) and their sums are added through LDS in order.
+template <int R, int WAVES>
+__global__ __launch_bounds__(kWave* WAVES) void gemv_n_shared_kernel(
+    const float* __restrict__ a, int64_t lda, const float* __restrict__ x, int64_t rows,
+    int64_t cols, float alpha, float beta, const float* __restrict__ y0, float* __restrict__ y) {
+    __shared__ double sums[WAVES][R];
+    constexpr int kInFlight = R == 1 ? 8 : 4; // loads per row and iteration
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
+    const float* arow[R];
+    double sum[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        sum[r] = 0.0;
+        arow[r] = a + (row0 + r < rows ? row0 + r : rows - 1) * lda;
+    }
+    const auto add = [&](float4 xv, const float4 (&av)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            sum[r] = fma(static_cast<double>(av[r].x), static_cast<double>(xv.x), sum[r]);
+            sum[r] = fma(static_cast<double>(av[r].y), static_cast<double>(xv.y), sum[r]);
+            sum[r] = fma(static_cast<double>(av[r].z), static_cast<double>(xv.z), sum[r]);
+            sum[r] = fma(static_cast<double>(av[r].w), static_cast<double>(xv.w), sum[r]);
+        }
+    };
+    const int64_t quads = cols / 4;
+    constexpr int64_t kStep = kWave * WAVES;
+    int64_t q = wave * kWave + lane;
+    for (; q + (kInFlight - 1) * kStep < quads; q += kInFlight * kStep) {
+        float4 xv[kInFlight], av[kInFlight][R];
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            xv[u] = mfr::dev::load_loose(x + 4 * (q + u * kStep));
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                av[u][r] = mfr::dev::load_streaming_loose(arow[r] + 4 * (q + u * kStep));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            add(xv[u], av[u]);
+        }
+    }
+#pragma unroll 2
+    for (; q < quads; q += kStep) {
+        float4 av[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            av[r] = mfr::dev::load_streaming_loose(arow[r] + 4 * q);
+        }
+        add(mfr::dev::load_loose(x + 4 * q), av);
+    }
+    const int64_t j = 4 * quads + lane; // the last 0 to 3 columns
+    if (wave == WAVES - 1 && j < cols) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            sum[r] = fma(static_cast<double>(arow[r][j]), static_cast<double>(x[j]), sum[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        sum[r] = mfr::dev::wave_sum(sum[r]);
+        if (lane == 0) {
+            sums[wave][r] = sum[r];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < R && row0 + threadIdx.x < rows) {
+        double total = sums[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) {
+            total += sums[w][threadIdx.x];
+        }
+        y[row0 + threadIdx.x] = finish(total, alpha, beta, y0, row0 + threadIdx.x);
+    }
+}
+
 constexpr int kStripCols = 256; // columns per workgroup in the T form: 64 lanes x 4
 constexpr int kUnrollT = 16;
 
 // Partial sums of one (column strip, row chunk) tile of A^T x: out[chunk][col], in double; one
-// wavefront, rows in increasing order. VEC4: lda % 4 == 0, cols % 4 == 0 and A 16-byte aligned,
-// so a lane's 4 columns are one float4; otherwise its columns are 64 apart.
-template <bool VEC4>
+// wavefront, rows in increasing order. QUADS: cols >= 4; a lane's 4 columns are adjacent and come
+// in one 16-byte load (4-byte aligned suffices), and lanes past the matrix take its last 4
+// columns (their sums repeat other lanes' bit for bit). Otherwise its columns are 64 apart.
+template <bool QUADS>
 __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
     const float* __restrict__ a, int64_t lda, const float* __restrict__ x, int64_t rows,
     int64_t cols, int64_t rows_per_chunk, double* __restrict__ partial) {
@@ -145,17 +225,19 @@ __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
     const int64_t chunk = blockIdx.y;
     const int64_t r_begin = chunk * rows_per_chunk;
     const int64_t r_end = r_begin + rows_per_chunk < rows ? r_begin + rows_per_chunk : rows;
-    // Column of component c of this lane: VEC4 -> 4 adjacent columns, else 4 columns 64 apart.
-    auto local_col = [&](int c) { return VEC4 ? 4 * lane + c : lane + c * kWave; };
-    const int64_t col_base = strip * kStripCols + local_col(0);
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    if constexpr (VEC4) {
-        const bool active = col_base < cols;
-        // A strip wholly inside the matrix (all but possibly the last) loads unconditionally;
-        // the condition is uniform across the wavefront.
-        const bool full_strip = (strip + 1) * kStripCols <= cols;
+    if constexpr (QUADS) {
+        int64_t col_base = strip * kStripCols + 4 * lane;
+        col_base = col_base + 4 <= cols ? col_base : cols - 4;
+        const auto add = [&](float4 av, float xf) {
+            const double xv = static_cast<double>(xf);
+            sum[0] = fma(static_cast<double>(av.x), xv, sum[0]);
+            sum[1] = fma(static_cast<double>(av.y), xv, sum[1]);
+            sum[2] = fma(static_cast<double>(av.z), xv, sum[2]);
+            sum[3] = fma(static_cast<double>(av.w), xv, sum[3]);
+        };
         int64_t r = r_begin;
-        if (full_strip && r + kUnrollT <= r_end) {
+        if (r + kUnrollT <= r_end) {
             // x[r .. r+15] is the same for every lane (a scalar load); it is fetched one
             // iteration ahead (index clamped to the last row) so its latency overlaps the
             // current iteration instead of stalling the stream of A loads.
@@ -168,7 +250,7 @@ __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
                 float4 av[kUnrollT];
 #pragma unroll
                 for (int u = 0; u < kUnrollT; ++u) {
-                    av[u] = mfr::dev::load_streaming(a + (r + u) * lda + col_base);
+                    av[u] = mfr::dev::load_streaming_loose(a + (r + u) * lda + col_base);
                 }
                 float xn[kUnrollT];
 #pragma unroll
@@ -178,11 +260,7 @@ __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
                 }
 #pragma unroll
                 for (int u = 0; u < kUnrollT; ++u) {
-                    const double xv = static_cast<double>(xr[u]);
-                    sum[0] = fma(static_cast<double>(av[u].x), xv, sum[0]);
-                    sum[1] = fma(static_cast<double>(av[u].y), xv, sum[1]);
-                    sum[2] = fma(static_cast<double>(av[u].z), xv, sum[2]);
-                    sum[3] = fma(static_cast<double>(av[u].w), xv, sum[3]);
+                    add(av[u], xr[u]);
                 }
 #pragma unroll
                 for (int u = 0; u < kUnrollT; ++u) {
@@ -190,15 +268,13 @@ __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
                 }
             }
         }
+#pragma unroll 4
         for (; r < r_end; ++r) {
-            const double xv = static_cast<double>(x[r]);
-            if (active) {
-                const float4 av = *reinterpret_cast<const float4*>(a + r * lda + col_base);
-                sum[0] = fma(static_cast<double>(av.x), xv, sum[0]);
-                sum[1] = fma(static_cast<double>(av.y), xv, sum[1]);
-                sum[2] = fma(static_cast<double>(av.z), xv, sum[2]);
-                sum[3] = fma(static_cast<double>(av.w), xv, sum[3]);
-            }
+            add(mfr::dev::load_streaming_loose(a + r * lda + col_base), x[r]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            partial[chunk * cols + col_base + c] = sum[c];
         }
     } else {
         for (int64_t r = r_begin; r < r_end; ++r) {
@@ -206,50 +282,83 @@ __global__ __launch_bounds__(kWave) void gemv_t_partial_kernel(
             const float* row = a + r * lda;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const int64_t col = strip * kStripCols + local_col(c);
+                const int64_t col = strip * kStripCols + lane + c * kWave;
                 if (col < cols) {
                     sum[c] = fma(static_cast<double>(row[col]), xv, sum[c]);
                 }
             }
         }
-    }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int64_t col = strip * kStripCols + local_col(c);
-        if (col < cols) {
-            partial[chunk * cols + col] = sum[c];
+        for (int c = 0; c < 4; ++c) {
+            const int64_t col = strip * kStripCols + lane + c * kWave;
+            if (col < cols) {
+                partial[chunk * cols + col] = sum[c];
+            }
         }
     }
 }
 
-// y[j] = finish(sum over chunks (in order) of partial[chunk][j]).
-__global__ void gemv_t_finish_kernel(const double* __restrict__ partial, int64_t chunks,
-                                     int64_t cols, float alpha, float beta,
-                                     const float* __restrict__ y0, float* __restrict__ y) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= cols) {
-        return;
-    }
+// y[j] = finish(sum over chunks of partial[chunk][j]): 4 wavefronts share 64 columns, each adding
+// a quarter of the chunks in order (8 loads in flight), then the quarters in order. One thread
+// adding every chunk of its column one load at a time took most of a 4093 x 1023 product's 86 us.
+constexpr int kFinishWaves = 4;
+__global__ __launch_bounds__(kWave* kFinishWaves) void gemv_t_finish_kernel(
+    const double* __restrict__ partial, int64_t chunks, int64_t cols, float alpha, float beta,
+    const float* __restrict__ y0, float* __restrict__ y) {
+    __shared__ double quarter[kFinishWaves][kWave];
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * kWave + lane;
+    const int64_t per = (chunks + kFinishWaves - 1) / kFinishWaves;
+    const int64_t first = wave * per;
+    const int64_t last = first + per < chunks ? first + per : chunks;
     double sum = 0.0;
-    for (int64_t c = 0; c < chunks; ++c) {
-        sum += partial[c * cols + j];
+    if (j < cols) {
+        int64_t c = first;
+        for (; c + 8 <= last; c += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                v[u] = partial[(c + u) * cols + j];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                sum += v[u];
+            }
+        }
+        for (; c < last; ++c) {
+            sum += partial[c * cols + j];
+        }
     }
-    y[j] = finish(sum, alpha, beta, y0, j);
+    quarter[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0 && j < cols) {
+#pragma unroll
+        for (int w = 1; w < kFinishWaves; ++w) {
+            sum += quarter[w][lane];
+        }
+        y[j] = finish(sum, alpha, beta, y0, j);
+    }
 }
 
 // Rows per chunk of the T form: about 2048 (strip, chunk) wavefronts (2 per SIMD of 256 CUs,
-// each with kUnrollT rows in flight), each chunk a multiple of the unrolled row step and at least
-// 64 rows.
+// each with kUnrollT rows in flight), each chunk a multiple of the unrolled row step.
 int64_t t_rows_per_chunk(int64_t rows, int64_t strips) {
     const int64_t target_tiles = 2048;
     int64_t chunks = (target_tiles + strips - 1) / strips;
     if (chunks < 1) {
         chunks = 1;
     }
-    int64_t per = (rows + chunks - 1) / chunks;
-    per = (per + kUnrollT - 1) / kUnrollT * kUnrollT;
-    return per < 64 ? 64 : per;
+    const int64_t per = (rows + chunks - 1) / chunks;
+    return (per + kUnrollT - 1) / kUnrollT * kUnrollT;
 }
+
+// The N form's kernel: the streaming kernel (8 rows per wavefront, aligned rows) where it gives
+// every CU 4 wavefronts; else from 2048 rows on 4 rows per workgroup (or 8 rows per wavefront
+// where the columns do not feed four of them: 16384 x 255 11.2 us with four), below that one.
+constexpr int64_t kStreamRows = 8192;
+constexpr int64_t kSharedRows = 2048;
+constexpr int64_t kNarrowCols = 512;
 
 void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float alpha,
                  const float* a, int64_t lda, const float* x, float beta, const float* y0,
@@ -268,13 +377,18 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
     const bool vec4 = mfr::aligned16(a) && lda % 4 == 0 && cols % 4 == 0 &&
                       (!trans ? mfr::aligned16(x) : true);
     if (!trans) {
-        const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
-        const unsigned blocks = mfr::grid_blocks(waves, kWavesPerBlockN);
-        if (vec4) {
-            gemv_n_kernel<true><<<blocks, kWave * kWavesPerBlockN, 0, s.stream>>>(
+        if (vec4 && rows >= kStreamRows) {
+            const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
+            gemv_n_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN), kWave * kWavesPerBlockN, 0,
+                            s.stream>>>(a, lda, x, rows, cols, alpha, beta, y0, y);
+        } else if (rows >= kSharedRows && cols <= kNarrowCols) {
+            gemv_n_shared_kernel<8, 1><<<mfr::grid_blocks(rows, 8), kWave, 0, s.stream>>>(
+                a, lda, x, rows, cols, alpha, beta, y0, y);
+        } else if (rows >= kSharedRows) {
+            gemv_n_shared_kernel<4, 4><<<mfr::grid_blocks(rows, 4), 4 * kWave, 0, s.stream>>>(
                 a, lda, x, rows, cols, alpha, beta, y0, y);
         } else {
-            gemv_n_kernel<false><<<blocks, kWave * kWavesPerBlockN, 0, s.stream>>>(
+            gemv_n_shared_kernel<1, 4><<<mfr::grid_blocks(rows, 1), 4 * kWave, 0, s.stream>>>(
                 a, lda, x, rows, cols, alpha, beta, y0, y);
         }
         mfr::check_launch("gemv_n_kernel");
@@ -292,7 +406,7 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
         partial = static_cast<double*>(
             s.reserve(static_cast<size_t>(chunks) * static_cast<size_t>(cols) * sizeof(double)));
         const dim3 grid(static_cast<unsigned>(strips), static_cast<unsigned>(chunks));
-        if (vec4) {
+        if (cols >= 4) {
             gemv_t_partial_kernel<true><<<grid, kWave, 0, s.stream>>>(
                 a, lda, x, rows, cols, per, partial);
         } else {
@@ -301,7 +415,7 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
         }
         mfr::check_launch("gemv_t_partial_kernel");
     }
-    gemv_t_finish_kernel<<<mfr::grid_blocks(cols, 256), 256, 0, s.stream>>>(
+    gemv_t_finish_kernel<<<mfr::grid_blocks(cols, kWave), kWave * kFinishWaves, 0, s.stream>>>(
         partial, chunks, cols, alpha, beta, y0, y);
     mfr::check_launch("gemv_t_finish_kernel");
 }
