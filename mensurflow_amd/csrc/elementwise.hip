@@ -499,6 +499,102 @@ __global__ __launch_bounds__(256) void softmax_rows_reg_kernel(const float* __re
     }
 }
 
+// Joins one value per wavefront through LDS: every thread gets op over all wavefronts' values, in
+// wavefront order. `slots` is free again after the next barrier.
+template <typename T, typename Op>
+__device__ __forceinline__ T join_waves(T v, T* slots, int waves, Op op) {
+    if (threadIdx.x % kWave == 0) {
+        slots[threadIdx.x / kWave] = v;
+    }
+    __syncthreads();
+    T all = slots[0];
+    for (int w = 1; w < waves; ++w) {
+        all = op(all, slots[w]);
+    }
+    return all;
+}
+
+// Softmax of long contiguous lines (a vocabulary's logits), one workgroup per line, the line held
+// in registers: thread t keeps the 4 adjacent values at 4 (t + THREADS i), i < QUADS, read and
+// written once in 16-byte accesses at any alignment. HBM-bound: 512 x 32003 (131 MB) took 600 us
+// with a wavefront walking each line three times, one value per lane and load.
+template <int THREADS, int QUADS>
+__global__ __launch_bounds__(THREADS) void softmax_block_kernel(const float* __restrict__ x,
+                                                                float* __restrict__ y,
+                                                                int64_t length) {
+    constexpr int kWaves = THREADS / kWave;
+    __shared__ float maxima[kWaves];
+    __shared__ double sums[kWaves];
+    const float* in = x + static_cast<int64_t>(blockIdx.x) * length;
+    float* out = y + static_cast<int64_t>(blockIdx.x) * length;
+    const int len = static_cast<int>(length);
+    float v[QUADS][4];
+    float m = -INFINITY;
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        const int j = 4 * (static_cast<int>(threadIdx.x) + THREADS * i);
+        if (j + 4 <= len) {
+            const float4 q = mfr::dev::load_loose(in + j);
+            v[i][0] = q.x;
+            v[i][1] = q.y;
+            v[i][2] = q.z;
+            v[i][3] = q.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[i][e] = j + e < len ? in[j + e] : -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            nan = nan || __builtin_isnan(v[i][e]);
+            m = fmaxf(m, v[i][e]);
+        }
+    }
+    // A NaN anywhere makes the maximum NaN: join it as +NaN, which the join keeps.
+    m = mfr::dev::wave_max(m);
+    m = __any(nan) ? NAN : m;
+    m = join_waves(m, maxima, kWaves, [](float p, float q) {
+        return __builtin_isnan(p) || __builtin_isnan(q) ? NAN : fmaxf(p, q);
+    });
+    double sum = 0.0;
+    if (m != -INFINITY) {
+#pragma unroll
+        for (int i = 0; i < QUADS; ++i) {
+            const int j = 4 * (static_cast<int>(threadIdx.x) + THREADS * i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[i][e] = expf(v[i][e] - m);
+                sum += j + e < len ? static_cast<double>(v[i][e]) : 0.0;
+            }
+        }
+    }
+    sum = join_waves(mfr::dev::wave_sum(sum), sums, kWaves, [](double p, double q) {
+        return p + q;
+    });
+    const float scale = static_cast<float>(1.0 / sum);
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        const int j = 4 * (static_cast<int>(threadIdx.x) + THREADS * i);
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e] = m == -INFINITY ? 0.0f : v[i][e] * scale; // every element masked out: zeros
+        }
+        if (j + 4 <= len) {
+            mfr::dev::store_loose(out + j, make_float4(o[0], o[1], o[2], o[3]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (j + e < len) {
+                    out[j + e] = o[e];
+                }
+            }
+        }
+    }
+}
+
 // Any line shape: one wavefront per line, three passes over the line in memory.
 __global__ __launch_bounds__(256) void softmax_lines_kernel(const float* __restrict__ x,
                                                             float* __restrict__ y, int64_t outer,
@@ -536,6 +632,64 @@ __global__ __launch_bounds__(256) void softmax_lines_kernel(const float* __restr
     const float scale = static_cast<float>(1.0 / sum);
     for (int64_t j = lane; j < length; j += kWave) {
         out[j * inner] = out[j * inner] * scale;
+    }
+}
+
+// argmax of wide rows, one workgroup per row: each thread takes 4 adjacent values per 16-byte load
+// (any alignment), 4 loads in flight, and keeps its best as a key that orders as the answer does:
+// the value's bits as an ordered integer (NaN above all, -0 as +0), then the lower index. Width
+// below 2^31. 512 x 32003: one wavefront per row left half the SIMDs idle and took 100 us.
+__device__ __forceinline__ uint64_t argmax_key(float v, uint32_t index) {
+    const uint32_t u = __float_as_uint(v + 0.0f); // -0 + 0 is +0
+    const uint32_t ordered = __builtin_isnan(v) ? 0xffffffffu
+                             : (u >> 31) != 0   ? ~u
+                                                : u | 0x80000000u;
+    return (static_cast<uint64_t>(ordered) << 32) | (0xffffffffu - index);
+}
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void argmax_block_kernel(const float* __restrict__ x,
+                                                               int64_t* __restrict__ out,
+                                                               int64_t width) {
+    constexpr int kWaves = THREADS / kWave;
+    constexpr int kInFlight = 4;
+    __shared__ uint64_t keys[kWaves];
+    const float* in = x + static_cast<int64_t>(blockIdx.x) * width;
+    const int len = static_cast<int>(width);
+    uint64_t best = 0;
+    const auto take = [&](float v, int j) {
+        const uint64_t key = argmax_key(v, static_cast<uint32_t>(j));
+        best = key > best ? key : best;
+    };
+    int j = 4 * static_cast<int>(threadIdx.x);
+    for (; j + 4 * THREADS * (kInFlight - 1) + 4 <= len; j += 4 * THREADS * kInFlight) {
+        float4 q[kInFlight];
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            q[u] = mfr::dev::load_loose(in + j + 4 * THREADS * u);
+        }
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            const int at = j + 4 * THREADS * u;
+            take(q[u].x, at);
+            take(q[u].y, at + 1);
+            take(q[u].z, at + 2);
+            take(q[u].w, at + 3);
+        }
+    }
+    for (; j < len; j += 4 * THREADS) {
+        for (int e = 0; e < 4 && j + e < len; ++e) {
+            take(in[j + e], j + e);
+        }
+    }
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) {
+        const uint64_t other = __shfl_xor(static_cast<unsigned long long>(best), offset, kWave);
+        best = other > best ? other : best;
+    }
+    best = join_waves(best, keys, kWaves, [](uint64_t p, uint64_t q) { return p > q ? p : q; });
+    if (threadIdx.x == 0) {
+        out[blockIdx.x] = static_cast<int64_t>(0xffffffffu - static_cast<uint32_t>(best));
     }
 }
 
@@ -898,12 +1052,24 @@ int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, in
             softmax_rows_reg_kernel<32, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
         } else if (inner == 1 && length <= 64 * 32) {
             softmax_rows_reg_kernel<32, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+        } else if (inner == 1 && length <= 4 * 256 * 8 && lines < (int64_t{1} << 31)) {
+            softmax_block_kernel<256, 8><<<static_cast<unsigned>(lines), 256, 0, s.stream>>>(
+                x, y, length);
+        } else if (inner == 1 && length <= 4 * 1024 * 4 && lines < (int64_t{1} << 31)) {
+            softmax_block_kernel<1024, 4><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
+                x, y, length);
+        } else if (inner == 1 && length <= 4 * 1024 * 8 && lines < (int64_t{1} << 31)) {
+            softmax_block_kernel<1024, 8><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
+                x, y, length);
         } else {
             softmax_lines_kernel<<<blocks, 256, 0, s.stream>>>(x, y, outer, length, inner);
         }
         mfr::check_launch("softmax_kernel");
     });
 }
+
+// Rows wider than this go a workgroup each.
+constexpr int64_t kArgmaxWide = 1024;
 
 int mfr_argmax(mfr_stream_t stream, const float* x, int64_t* out, int64_t rows, int64_t width) {
     return mfr::guarded([&] {
@@ -913,7 +1079,17 @@ int mfr_argmax(mfr_stream_t stream, const float* x, int64_t* out, int64_t rows, 
             return;
         }
         mfr::require(out != nullptr && (width == 0 || x != nullptr), "argmax: null pointer");
-        argmax_kernel<<<mfr::grid_blocks(rows, 4), 256, 0, s.stream>>>(x, out, rows, width);
+        if (width > kArgmaxWide && width < (int64_t{1} << 31) - 65536 &&
+            rows < (int64_t{1} << 31)) {
+            const unsigned grid = static_cast<unsigned>(rows);
+            if (width <= 8192) {
+                argmax_block_kernel<256><<<grid, 256, 0, s.stream>>>(x, out, width);
+            } else {
+                argmax_block_kernel<1024><<<grid, 1024, 0, s.stream>>>(x, out, width);
+            }
+        } else {
+            argmax_kernel<<<mfr::grid_blocks(rows, 4), 256, 0, s.stream>>>(x, out, rows, width);
+        }
         mfr::check_launch("argmax_kernel");
     });
 }
