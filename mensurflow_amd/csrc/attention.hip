@@ -24,6 +24,8 @@
 //     16-byte rows.
 //   - attention16_kernel (below) is the same op with 16 queries per wavefront on the 16x16x4
 //     MFMA, at 4 wavefronts per SIMD; it takes causal d = 64 on large grids.
+//   - At most 4 queries go to the decode form (attention_decode.hip).
+#include "attention.hpp"
 #include "gemm_kernel.hpp"
 
 #include <cmath>
@@ -56,26 +58,7 @@ int waves_used(int64_t d, int64_t lq, int64_t batch_count, bool causal, int cus)
 }
 constexpr float kLog2e = 1.4426950408889634f;
 
-struct AttnParams {
-    const float* q;
-    const float* k;
-    const float* v;
-    float* out;
-    const uint8_t* mask;
-    int64_t lq, lk;
-    int64_t q_rs, k_rs, v_rs, out_rs, mask_rs, mask_cs;
-    int64_t batch[MFR_MAX_BATCH_DIMS];
-    int64_t q_bs[MFR_MAX_BATCH_DIMS], k_bs[MFR_MAX_BATCH_DIMS], v_bs[MFR_MAX_BATCH_DIMS];
-    int64_t out_bs[MFR_MAX_BATCH_DIMS], mask_bs[MFR_MAX_BATCH_DIMS];
-    int64_t batch_count;
-    int32_t batch_dims;
-    int32_t causal;
-    int32_t q_blocks;
-    // Issue order of the query blocks: longest first, or (paired) the longer half longest first,
-    // then the shorter half shortest first.
-    int32_t paired;
-    float scale;
-};
+using mfr::attn::AttnParams;
 
 // Which (batch entry, query block) workgroup blockIdx.x computes, and that entry's element
 // offsets into q, k, v, out and the mask. Query blocks are issued longest first (the last ones of
@@ -896,6 +879,10 @@ void run_attention(mfr_stream& s, const mfr_attention_desc& d) {
     p.causal = d.causal != 0;
     p.scale = d.scale != 0.0f ? d.scale
                               : static_cast<float>(1.0 / std::sqrt(static_cast<double>(d.d)));
+    if (d.lq <= mfr::attn::kDecodeMaxQueries && d.lk > 0) {
+        mfr::attn::run_decode(s, p, d.d);
+        return;
+    }
     const int waves = waves_used(d.d, d.lq, batch_count, d.causal != 0, s.compute_units);
     // d = 64, causal, no mask, a grid of 8-wavefront workgroups: the 16-query kernel, whose
     // last diagonal key blocks keep every SIMD busy (configs[4]: 163.6 against 170.0 us).

@@ -1,0 +1,73 @@
+"""Attention of 1 to 4 queries (the decode form): key counts around a wavefront's and a range's
+edges, every head size, masks, causal, broadcast keys, NaN and fully masked rows, against float64
+with the fused kernel's bound 1e-5 * sqrt(lk) of sum_j |p_ij v_jc|."""
+import numpy as np
+import pytest
+
+import mensurflow_amd as mf
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, keep):
+    """Output and its magnitude sum_j p_ij |v_jc| in float64; keep [.., lq, lk] of booleans."""
+    q, k, v = (t.astype(np.float64) for t in (q, k, v))
+    s = q @ np.swapaxes(k, -1, -2) / np.sqrt(q.shape[-1])
+    s = np.where(keep, s, -np.inf)
+    top = np.max(s, axis=-1, keepdims=True)
+    p = np.exp(s - np.where(np.isfinite(top), top, 0.0))
+    total = p.sum(axis=-1, keepdims=True)
+    p = np.divide(p, total, out=np.zeros_like(p), where=total > 0)
+    return p @ v, p @ np.abs(v)
+
+
+def check(stream, batch, lq, lk, d, causal=False, masked=False, broadcast=False, seed=0):
+    rng = np.random.default_rng(seed)
+    kv_batch = (batch[0],) + (1,) * (len(batch) - 1) if broadcast else batch
+    q = rng.standard_normal(batch + (lq, d)).astype(np.float32)
+    k = rng.standard_normal(kv_batch + (lk, d)).astype(np.float32)
+    v = rng.standard_normal(kv_batch + (lk, d)).astype(np.float32)
+    keep = np.ones(batch + (lq, lk), bool)
+    mask_d = None
+    if masked:
+        keep = rng.random(batch + (lq, lk)) < 0.6
+        keep[..., 0, :] = False  # a fully masked row
+        mask_d = mf.DeviceArray.from_numpy(keep.astype(np.uint8), stream)
+    if causal:
+        keep = keep & np.tril(np.ones((lq, lk), bool))
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    got = mf.attention_fused(dev(q), dev(k).expand(batch + (lk, d)), dev(v).expand(batch + (lk, d)),
+                             mask=mask_d, causal=causal).numpy()
+    want, scale = reference(q, k, v, keep)
+    bound = 1e-5 * np.sqrt(lk) * scale
+    assert np.all(np.abs(got - want) <= bound), (batch, lq, lk, d, causal, masked)
+
+
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize("lq,lk", [(1, 1), (1, 7), (1, 255), (2, 256), (3, 257), (4, 1000),
+                                   (1, 4097), (4, 16384)])
+def test_head_sizes_and_key_counts(stream, d, lq, lk):
+    check(stream, (2, 3), lq, lk, d, seed=d + lk)
+
+
+@pytest.mark.parametrize("lq,lk", [(1, 33), (2, 300), (4, 2049)])
+def test_masks_causal_broadcast(stream, lq, lk):
+    for d in (32, 64, 128):
+        check(stream, (2, 3), lq, lk, d, causal=True, seed=1)
+        check(stream, (2, 3), lq, lk, d, masked=True, seed=2)
+        check(stream, (2, 4), lq, lk, d, masked=True, causal=True, broadcast=True, seed=3)
+    check(stream, (300, 5), lq, lk, 64, seed=4)  # as many heads as ranges fill the chip: one range
+    check(stream, (), lq, lk, 64, seed=5)
+
+
+def test_nan_and_infinite_keys(stream):
+    """A NaN score makes its row NaN and leaves other rows alone, in the last range too."""
+    for lk in (100, 5000):
+        rng = np.random.default_rng(lk)
+        q, k, v = (rng.standard_normal((3, n, 64)).astype(np.float32) for n in (2, lk, lk))
+        k[1, lk - 1, 5] = np.nan
+        dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+        got = mf.attention_fused(dev(q), dev(k), dev(v)).numpy()
+        assert np.all(np.isnan(got[1])) and np.all(np.isfinite(got[[0, 2]]))
+        want, scale = reference(q, k, v, np.ones((3, 2, lk), bool))
+        assert np.all(np.abs(got - want)[[0, 2]] <= 1e-5 * np.sqrt(lk) * scale[[0, 2]])
