@@ -209,6 +209,43 @@ __global__ __launch_bounds__(kWave* WAVES) void gemv_n_shared_kernel(
     }
 }
 
+// N form for many short rows at any alignment (cols <= kNarrowCols): 8 rows per wavefront, one
+// float per lane and load, the 8 rows' loads together (16384 x 255 5.4 us, 12000 x 333 5.0; as
+// gemv_n_shared_kernel 11.2 and 9.1).
+__global__ __launch_bounds__(kWave* kWavesPerBlockN) void gemv_n_narrow_kernel(
+    const float* __restrict__ a, int64_t lda, const float* __restrict__ x, int64_t rows,
+    int64_t cols, float alpha, float beta, const float* __restrict__ y0, float* __restrict__ y) {
+    const int lane = threadIdx.x % kWave;
+    const int64_t wave = static_cast<int64_t>(blockIdx.x) * kWavesPerBlockN + threadIdx.x / kWave;
+    const int64_t row0 = wave * kRowsPerWave;
+    if (row0 >= rows) {
+        return;
+    }
+    const float* arow[kRowsPerWave];
+    double sum[kRowsPerWave];
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+        sum[r] = 0.0;
+        arow[r] = a + (row0 + r < rows ? row0 + r : rows - 1) * lda;
+    }
+    for (int64_t j = lane; j < cols; j += kWave) {
+        const double xj = static_cast<double>(x[j]);
+#pragma unroll
+        for (int r = 0; r < kRowsPerWave; ++r) {
+            sum[r] = fma(static_cast<double>(arow[r][j]), xj, sum[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+        sum[r] = mfr::dev::wave_sum(sum[r]);
+    }
+    if (lane == 0) {
+        for (int r = 0; r < kRowsPerWave && row0 + r < rows; ++r) {
+            y[row0 + r] = finish(sum[r], alpha, beta, y0, row0 + r);
+        }
+    }
+}
+
 constexpr int kStripCols = 256; // columns per workgroup in the T form: 64 lanes x 4
 constexpr int kUnrollT = 16;
 
@@ -354,8 +391,8 @@ int64_t t_rows_per_chunk(int64_t rows, int64_t strips) {
 }
 
 // The N form's kernel: the streaming kernel (8 rows per wavefront, aligned rows) where it gives
-// every CU 4 wavefronts; else from 2048 rows on 4 rows per workgroup (or 8 rows per wavefront
-// where the columns do not feed four of them: 16384 x 255 11.2 us with four), below that one.
+// every CU 4 wavefronts; else from 2048 rows on 4 rows per workgroup (or the narrow kernel where
+// the columns do not feed four wavefronts), below that one.
 constexpr int64_t kStreamRows = 8192;
 constexpr int64_t kSharedRows = 2048;
 constexpr int64_t kNarrowCols = 512;
@@ -382,7 +419,9 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
             gemv_n_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN), kWave * kWavesPerBlockN, 0,
                             s.stream>>>(a, lda, x, rows, cols, alpha, beta, y0, y);
         } else if (rows >= kSharedRows && cols <= kNarrowCols) {
-            gemv_n_shared_kernel<8, 1><<<mfr::grid_blocks(rows, 8), kWave, 0, s.stream>>>(
+            const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
+            gemv_n_narrow_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN),
+                                   kWave * kWavesPerBlockN, 0, s.stream>>>(
                 a, lda, x, rows, cols, alpha, beta, y0, y);
         } else if (rows >= kSharedRows) {
             gemv_n_shared_kernel<4, 4><<<mfr::grid_blocks(rows, 4), 4 * kWave, 0, s.stream>>>(
