@@ -1,0 +1,93 @@
+"""The fused attention on the bf16 matrix cores where its parts could miss the fp32 values: infinite,
+NaN, huge and tiny operands, in the first and the last key block, causal and masked, for every head
+size and both workgroup sizes; against float64 with the fused kernel's bound."""
+import numpy as np
+import pytest
+
+import mensurflow_amd as mf
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, keep):
+    with np.errstate(all="ignore"):
+        s = q.astype(np.float64) @ np.swapaxes(k.astype(np.float64), -1, -2) / np.sqrt(q.shape[-1])
+        s = np.where(keep, s, -np.inf)
+        top = np.max(s, axis=-1, keepdims=True)
+        p = np.exp(s - np.where(top == -np.inf, 0.0, top))
+        total = p.sum(axis=-1, keepdims=True)
+        p = np.where(total == 0, 0.0, p / total)
+        out = np.zeros(q.shape[:-1] + (v.shape[-1],))
+        mag = np.zeros_like(out)
+        # A removed key adds nothing here; the weight 0 of a kept one still meets its value.
+        for idx in np.ndindex(q.shape[:-2]):
+            out[idx] = p[idx] @ v[idx].astype(np.float64)
+            mag[idx] = p[idx] @ np.abs(v[idx].astype(np.float64))
+    return out, mag
+
+
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("case", ["value inf", "value nan", "key -inf", "key nan", "huge value",
+                                  "tiny values", "huge scores"])
+def test_extreme_operands(stream, d, case):
+    for batch, lq, lk, causal in (((2,), 70, 150, False), ((2,), 260, 260, True),
+                                  ((70, 4), 300, 64, False)):
+        rng = np.random.default_rng(d)
+        q = rng.standard_normal(batch + (lq, d)).astype(np.float32)
+        k = rng.standard_normal(batch + (lk, d)).astype(np.float32)
+        v = rng.standard_normal(batch + (lk, d)).astype(np.float32)
+        one = (0,) * len(batch)
+        if case == "value inf":
+            v[one + (0, 3)] = np.inf   # kept by every query
+        elif case == "value nan":
+            v[one + (0, d - 1)] = np.nan
+        elif case == "key -inf":
+            q[..., 0] = np.abs(q[..., 0]) + 0.1
+            k[one + (5, 0)] = -np.inf  # a weight of 0
+        elif case == "key nan":
+            k[one + (0, 1)] = np.nan
+        elif case == "huge value":
+            v[one + (0, slice(None))] = 3.4e38  # above the largest bf16
+            v[one + (slice(1, None), slice(None))] = 0.0
+        elif case == "tiny values":
+            v *= np.float32(1e-37)
+        elif case == "huge scores":
+            q *= np.float32(1e18)
+            k *= np.float32(1e18)
+        keep = np.tril(np.ones((lq, lk), bool)) if causal else np.ones((lq, lk), bool)
+        dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+        got = mf.attention_fused(dev(q), dev(k), dev(v), causal=causal).numpy()
+        want, mag = reference(q, k, v, keep)
+        what = (case, d, batch, lq, lk)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), what
+        ok = np.isfinite(want)
+        assert np.array_equal(got[~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)]), what
+        if case != "huge scores":  # there the scores' own rounding moves the weights
+            bound = 1e-5 * np.sqrt(lk) * mag + lk * 2.0**-149
+            assert np.all(np.abs(got[ok] - want[ok]) <= bound[ok]), what
+
+
+@pytest.mark.parametrize("form", ["row", "rows", "strided"])
+def test_mask_forms(stream, form):
+    """A mask row shared by all queries, a row each, and a row whose bytes are not adjacent, with
+    key counts around the 4-byte words and the 32-key blocks."""
+    for d in (32, 64, 128):
+        for lk in (5, 32, 63, 97, 130):
+            rng = np.random.default_rng(lk)
+            b, lq = 3, 40
+            q, k, v = (rng.standard_normal((b, n, d)).astype(np.float32) for n in (lq, lk, lk))
+            dev = lambda x: mf.DeviceArray.from_numpy(np.ascontiguousarray(x), stream)  # noqa: E731
+            if form == "row":
+                keep = rng.random((b, 1, lk)) < 0.5
+                mask = dev(keep.astype(np.uint8))
+            elif form == "rows":
+                keep = rng.random((b, lq, lk)) < 0.5
+                keep[:, 3] = False
+                mask = dev(keep.astype(np.uint8))
+            else:
+                keep = rng.random((b, lq, lk)) < 0.5
+                mask = dev(np.swapaxes(keep, 1, 2).astype(np.uint8)).T
+            full = np.broadcast_to(keep, (b, lq, lk))
+            got = mf.attention_fused(dev(q), dev(k), dev(v), mask=mask).numpy()
+            want, mag = reference(q, k, v, full)
+            assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * mag), (form, d, lk)
