@@ -89,6 +89,7 @@ constexpr int kMaxSplits = MFR_MAX_SPLITS;
 constexpr double kMaxPartialBytes = 1073741824.0; // AUTO keeps the partial sums under 1 GiB
 constexpr double kReduceBytesPerUs = 3.7e6;       // split_reduce_kernel's HBM rate (bytes/us)
 constexpr double kReduceLaunchUs = 2.4;           // its launch and ramp
+constexpr double kReduceSumUs = 0.15;             // each range past 8 a thread adds in turn
 
 // AUTO never cuts a range shorter than this: two slices more than a tile's fixed time is worth.
 constexpr int64_t min_auto_depth(int tile) { return tile == MFR_TILE_64x64 ? 128 : 256; }
@@ -105,6 +106,8 @@ int splits_for(int64_t k, int64_t per) { return static_cast<int>((k + per - 1) /
 // form (sgemm_split_regs_kernel): every CU has at most one workgroup, and either more than half
 // of them have one or the depth is short; AUTO splits a longer depth over the idle CUs. 1024^3
 // 24.8 -> 20.7 us.
+constexpr int64_t kFewRows = 32; // at most this many rows run its 32x64 form, split or not
+
 bool regs_form(int64_t count, int64_t k, int cus) {
     return count <= cus && (2 * count > cus || k <= 512);
 }
@@ -120,7 +123,8 @@ double modelled_us(int t, int64_t m, int64_t n, int64_t k, int64_t batch, int cu
     const int64_t count = tile_count(t, m, n, batch) * splits;
     const int64_t per_cu = (count + cus - 1) / cus;
     const int64_t resident = per_cu < info.occupancy ? per_cu : info.occupancy;
-    const bool regs = t == MFR_TILE_64x64 && splits == 1 && regs_form(count, k, cus);
+    const bool regs = t == MFR_TILE_64x64 &&
+                      (m <= kFewRows || (splits == 1 && regs_form(count, k, cus)));
     const double depth = static_cast<double>(splits > 1 ? per : k);
     const double tile_us = regs ? kRegsDepthUs * depth + kRegsFixedUs
                                 : info.depth_us[resident - 1] * depth +
@@ -131,7 +135,7 @@ double modelled_us(int t, int64_t m, int64_t n, int64_t k, int64_t batch, int cu
     if (splits > 1) {
         const double outputs = static_cast<double>(m) * n * batch;
         us += outputs * 4.0 * (2.0 * splits + (c0 ? 2.0 : 1.0)) / kReduceBytesPerUs +
-              kReduceLaunchUs;
+              kReduceLaunchUs + kReduceSumUs * std::max(0, splits - 8);
     }
     return us;
 }
@@ -372,7 +376,9 @@ void launch_split(int tile, const GemmParams& q, bool ak, bool bk, unsigned bloc
     case MFR_TILE_128x64: launch_split_128x64(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x128: launch_split_64x128(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x64:
-        if (q.splits == 1 && regs_form(blocks, q.k, cus) && near) {
+        if (q.m <= kFewRows && near) {
+            launch_split_regs_32x64(q, ak, bk, blocks, stream);
+        } else if (q.splits == 1 && regs_form(blocks, q.k, cus) && near) {
             launch_split_regs_64x64(q, ak, bk, blocks, stream);
         } else {
             launch_split_64x64(q, ak, bk, blocks, stream);

@@ -13,6 +13,9 @@ void launch_split_64x128(const GemmParams& p, bool ak, bool bk, unsigned blocks,
 // No LDS in the depth loop; M/N-major lines less than 2^26 floats apart.
 void launch_split_regs_64x64(const GemmParams& p, bool ak, bool bk, unsigned blocks,
                              hipStream_t s);
+// Likewise, on 64x64 tiles of which at most 32 rows are inside the matrix.
+void launch_split_regs_32x64(const GemmParams& p, bool ak, bool bk, unsigned blocks,
+                             hipStream_t s);
 void launch_split_64x64(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
 
 } // namespace mfr::gemm

@@ -532,8 +532,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
 
 // One operand's share of a 16-deep step for a wavefront of the register form: F blocks of 32 rows,
 // lane l the 8 depths 8 (l / 32) .. of row l % 32 of each, which are its MFMA fragments.
-template <int F, bool KMAJ> struct StepLoader {
-    float reg[F][8];
+template <int F, bool KMAJ, int SETS = 1> struct StepLoader {
+    float reg[SETS][F][8]; // a step in flight each
     const float* at[KMAJ ? F : 1]; // K-major: this lane's depths in the wavefront's next step
     const float* line;             // M/N-major: the next step's first depth line
     int64_t stride;
@@ -558,8 +558,8 @@ template <int F, bool KMAJ> struct StepLoader {
     }
 
     // Loads a step (whole, or k_left depths of it) and moves on by `steps` steps.
-    template <bool WHOLE> __device__ __forceinline__ void load(int64_t k_left, int steps,
-                                                               int half) {
+    template <bool WHOLE> __device__ __forceinline__ void load(int set, int64_t k_left,
+                                                               int steps, int half) {
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             if constexpr (WHOLE && KMAJ) {
@@ -568,20 +568,20 @@ template <int F, bool KMAJ> struct StepLoader {
                 const native4 hi = *reinterpret_cast<const loose4*>(at[f] + 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    reg[f][e] = lo[e];
-                    reg[f][4 + e] = hi[e];
+                    reg[set][f][e] = lo[e];
+                    reg[set][f][4 + e] = hi[e];
                 }
             } else if constexpr (WHOLE) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    reg[f][e] = (line + e * stride)[offset[f]];
+                    reg[set][f][e] = (line + e * stride)[offset[f]];
                 }
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    reg[f][e] = 0.0f;
+                    reg[set][f][e] = 0.0f;
                     if (8 * half + e < k_left) {
-                        reg[f][e] = KMAJ ? at[KMAJ ? f : 0][e]
+                        reg[set][f][e] = KMAJ ? at[KMAJ ? f : 0][e]
                                          : (line + e * stride)[offset[KMAJ ? 0 : f]];
                     }
                 }
@@ -594,11 +594,12 @@ template <int F, bool KMAJ> struct StepLoader {
         line += KMAJ ? 0 : 16 * steps * stride;
     }
 
-    __device__ __forceinline__ void cut(bf16x8 (&part)[F][3], float& squares) const {
+    __device__ __forceinline__ void cut(int set, bf16x8 (&part)[F][3],
+                                        float& squares) const {
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             uint32_t words[3][4];
-            cut_eight(reg[f], words, squares);
+            cut_eight(reg[set][f], words, squares);
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 part[f][q] = __builtin_bit_cast(
@@ -613,7 +614,7 @@ template <int F, bool KMAJ> struct StepLoader {
         for (int f = 0; f < F; ++f) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                least = min(least, (__float_as_uint(reg[f][e]) & 0x7fffffffu) - 1);
+                least = min(least, (__float_as_uint(reg[0][f][e]) & 0x7fffffffu) - 1);
             }
         }
         return least;
@@ -628,8 +629,12 @@ template <int F, bool KMAJ> struct StepLoader {
 // The same cuts and MFMAs as the LDS form, but no barrier holds the wavefronts in step and every
 // MFMA has independent ones beside it, which counts where a CU has one workgroup: 1024^3 24.8 ->
 // 20.7 us. With several workgroups per CU the LDS form is faster (2048 x 2048 x 1024: 58.8 us
-// against 67 with 4 sets and 76 with 8).
-template <int BM, int BN, int WAVES_K, bool AK, bool BK>
+// against 67 with 4 sets and 76 with 8). SETS steps are in flight in registers: 1 for 64x64, 2 for
+// 32x64 (the first 32 rows of a 64x64 tile: a few rows against a large matrix, 32 x 4096 x 4096
+// 25.3 -> 22.6 us). 32-deep steps (a whole 128-byte line of a K-major row each) took 1024^3 from
+// 19.7 to 25.3 us, and 32x32 tiles of 16 sets over the whole depth, which need no reduce, 35.8 us
+// at 32 x 4096 x 4096.
+template <int BM, int BN, int WAVES_K, int SETS, bool AK, bool BK>
 __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmParams p) {
     constexpr int FM = BM / 32, FN = BN / 32;
     constexpr int kBlocks = FM * FN;
@@ -669,27 +674,28 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
     }
     float squares = 0.0f;
     {
-        StepLoader<FM, AK> la(a_base, p.a_rs, p.a_cs, w.rows_a, set, half, r32);
-        StepLoader<FN, BK> lb(b_base, p.b_cs, p.b_rs, w.rows_b, set, half, r32);
-        const auto load = [&](int64_t t) __attribute__((always_inline)) {
+        StepLoader<FM, AK, SETS> la(a_base, p.a_rs, p.a_cs, w.rows_a, set, half, r32);
+        StepLoader<FN, BK, SETS> lb(b_base, p.b_cs, p.b_rs, w.rows_b, set, half, r32);
+        const auto load = [&](int into, int64_t t) __attribute__((always_inline)) {
             const int64_t k_left = kk - 16 * t;
             if (k_left >= 16) {
-                la.template load<true>(k_left, WAVES_K, half);
-                lb.template load<true>(k_left, WAVES_K, half);
+                la.template load<true>(into, k_left, WAVES_K, half);
+                lb.template load<true>(into, k_left, WAVES_K, half);
             } else if (k_left > 0) {
-                la.template load<false>(k_left, WAVES_K, half);
-                lb.template load<false>(k_left, WAVES_K, half);
+                la.template load<false>(into, k_left, WAVES_K, half);
+                lb.template load<false>(into, k_left, WAVES_K, half);
             }
         };
-        const auto step = [&](auto whole, int64_t t) __attribute__((always_inline)) {
+        // Step t, loaded into register set `from`, which then takes step t + SETS WAVES_K.
+        const auto step = [&](auto whole, int from, int64_t t) __attribute__((always_inline)) {
             bf16x8 fa[FM][3], fb[FN][3];
-            la.cut(fa, squares);
-            lb.cut(fb, squares);
+            la.cut(from, fa, squares);
+            lb.cut(from, fb, squares);
             if constexpr (decltype(whole)::value) {
-                la.template load<true>(16, WAVES_K, half);
-                lb.template load<true>(16, WAVES_K, half);
+                la.template load<true>(from, 16, WAVES_K, half);
+                lb.template load<true>(from, 16, WAVES_K, half);
             } else {
-                load(t + WAVES_K);
+                load(from, t + SETS * WAVES_K);
             }
 #pragma unroll
             for (int q = 0; q < 6; ++q) {
@@ -704,14 +710,23 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
             }
         };
         int64_t t = set;
-        if (t < steps) {
-            load(t);
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) {
+            load(i, t + i * WAVES_K);
         }
-        for (; 16 * (t + WAVES_K + 1) <= kk; t += WAVES_K) {
-            step(std::true_type{}, t);
+        for (; 16 * (t + (2 * SETS - 1) * WAVES_K + 1) <= kk; t += SETS * WAVES_K) {
+#pragma unroll
+            for (int i = 0; i < SETS; ++i) {
+                step(std::true_type{}, i, t + i * WAVES_K);
+            }
         }
-        for (; t < steps; t += WAVES_K) {
-            step(std::false_type{}, t);
+        for (; t < steps; t += SETS * WAVES_K) {
+#pragma unroll
+            for (int i = 0; i < SETS; ++i) {
+                if (t + i * WAVES_K < steps) {
+                    step(std::false_type{}, i, t + i * WAVES_K);
+                }
+            }
         }
     }
     squares = mfr::dev::butterfly_sum(squares);
@@ -769,11 +784,11 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
         for (int64_t t = set; t < steps; t += WAVES_K) {
             const int64_t k_left = kk - 16 * t;
             if (k_left >= 16) {
-                ra.template load<true>(k_left, WAVES_K, half);
-                rb.template load<true>(k_left, WAVES_K, half);
+                ra.template load<true>(0, k_left, WAVES_K, half);
+                rb.template load<true>(0, k_left, WAVES_K, half);
             } else {
-                ra.template load<false>(k_left, WAVES_K, half);
-                rb.template load<false>(k_left, WAVES_K, half);
+                ra.template load<false>(0, k_left, WAVES_K, half);
+                rb.template load<false>(0, k_left, WAVES_K, half);
             }
             found = min(found, min(ra.smallest(), rb.smallest()));
         }
@@ -811,18 +826,18 @@ void launch_split_tile(const GemmParams& p, bool ak, bool bk, unsigned blocks,
     }
 }
 
-template <int BM, int BN, int WAVES_K>
+template <int BM, int BN, int WAVES_K, int SETS>
 void launch_split_regs_tile(const GemmParams& p, bool ak, bool bk, unsigned blocks,
                             hipStream_t stream) {
     constexpr unsigned threads = WAVES_K * 64;
     if (ak && bk) {
-        sgemm_split_regs_kernel<BM, BN, WAVES_K, true, true><<<blocks, threads, 0, stream>>>(p);
+        sgemm_split_regs_kernel<BM, BN, WAVES_K, SETS, true, true><<<blocks, threads, 0, stream>>>(p);
     } else if (ak) {
-        sgemm_split_regs_kernel<BM, BN, WAVES_K, true, false><<<blocks, threads, 0, stream>>>(p);
+        sgemm_split_regs_kernel<BM, BN, WAVES_K, SETS, true, false><<<blocks, threads, 0, stream>>>(p);
     } else if (bk) {
-        sgemm_split_regs_kernel<BM, BN, WAVES_K, false, true><<<blocks, threads, 0, stream>>>(p);
+        sgemm_split_regs_kernel<BM, BN, WAVES_K, SETS, false, true><<<blocks, threads, 0, stream>>>(p);
     } else {
-        sgemm_split_regs_kernel<BM, BN, WAVES_K, false, false><<<blocks, threads, 0, stream>>>(p);
+        sgemm_split_regs_kernel<BM, BN, WAVES_K, SETS, false, false><<<blocks, threads, 0, stream>>>(p);
     }
 }
 
