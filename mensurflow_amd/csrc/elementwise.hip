@@ -1028,6 +1028,9 @@ int mfr_where_nd(mfr_stream_t stream, int32_t ndim, const int64_t* shape, const 
     });
 }
 
+// A workgroup of up to 1024 threads per row, fewer than 2^32 threads in a launch.
+constexpr int64_t kBlockRows = int64_t{1} << 22;
+
 int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, int64_t length,
                 int64_t inner) {
     return mfr::guarded([&] {
@@ -1052,13 +1055,13 @@ int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, in
             softmax_rows_reg_kernel<32, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
         } else if (inner == 1 && length <= 64 * 32) {
             softmax_rows_reg_kernel<32, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 4 * 256 * 8 && lines < (int64_t{1} << 31)) {
+        } else if (inner == 1 && length <= 4 * 256 * 8 && lines < kBlockRows) {
             softmax_block_kernel<256, 8><<<static_cast<unsigned>(lines), 256, 0, s.stream>>>(
                 x, y, length);
-        } else if (inner == 1 && length <= 4 * 1024 * 4 && lines < (int64_t{1} << 31)) {
+        } else if (inner == 1 && length <= 4 * 1024 * 4 && lines < kBlockRows) {
             softmax_block_kernel<1024, 4><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
                 x, y, length);
-        } else if (inner == 1 && length <= 4 * 1024 * 8 && lines < (int64_t{1} << 31)) {
+        } else if (inner == 1 && length <= 4 * 1024 * 8 && lines < kBlockRows) {
             softmax_block_kernel<1024, 8><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
                 x, y, length);
         } else {
@@ -1080,7 +1083,7 @@ int mfr_argmax(mfr_stream_t stream, const float* x, int64_t* out, int64_t rows, 
         }
         mfr::require(out != nullptr && (width == 0 || x != nullptr), "argmax: null pointer");
         if (width > kArgmaxWide && width < (int64_t{1} << 31) - 65536 &&
-            rows < (int64_t{1} << 31)) {
+            rows < kBlockRows) {
             const unsigned grid = static_cast<unsigned>(rows);
             if (width <= 8192) {
                 argmax_block_kernel<256><<<grid, 256, 0, s.stream>>>(x, out, width);

@@ -345,36 +345,41 @@ __global__ __launch_bounds__(kWave* kFinishWaves) void gemv_t_finish_kernel(
     __shared__ double quarter[kFinishWaves][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * kWave + lane;
     const int64_t per = (chunks + kFinishWaves - 1) / kFinishWaves;
     const int64_t first = wave * per;
     const int64_t last = first + per < chunks ? first + per : chunks;
-    double sum = 0.0;
-    if (j < cols) {
-        int64_t c = first;
-        for (; c + 8 <= last; c += 8) {
-            double v[8];
+    // Uniform: every thread of the workgroup takes the same blocks of 64 columns.
+    for (int64_t block = static_cast<int64_t>(blockIdx.x) * kWave; block < cols;
+         block += static_cast<int64_t>(gridDim.x) * kWave) {
+        const int64_t j = block + lane;
+        double sum = 0.0;
+        if (j < cols) {
+            int64_t c = first;
+            for (; c + 8 <= last; c += 8) {
+                double v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                v[u] = partial[(c + u) * cols + j];
+                for (int u = 0; u < 8; ++u) {
+                    v[u] = partial[(c + u) * cols + j];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    sum += v[u];
+                }
             }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                sum += v[u];
+            for (; c < last; ++c) {
+                sum += partial[c * cols + j];
             }
         }
-        for (; c < last; ++c) {
-            sum += partial[c * cols + j];
-        }
-    }
-    quarter[wave][lane] = sum;
-    __syncthreads();
-    if (wave == 0 && j < cols) {
+        quarter[wave][lane] = sum;
+        __syncthreads();
+        if (wave == 0 && j < cols) {
 #pragma unroll
-        for (int w = 1; w < kFinishWaves; ++w) {
-            sum += quarter[w][lane];
+            for (int w = 1; w < kFinishWaves; ++w) {
+                sum += quarter[w][lane];
+            }
+            y[j] = finish(sum, alpha, beta, y0, j);
         }
-        y[j] = finish(sum, alpha, beta, y0, j);
+        __syncthreads(); // `quarter` has been read
     }
 }
 
@@ -396,6 +401,7 @@ int64_t t_rows_per_chunk(int64_t rows, int64_t strips) {
 constexpr int64_t kStreamRows = 8192;
 constexpr int64_t kSharedRows = 2048;
 constexpr int64_t kNarrowCols = 512;
+constexpr int64_t kManyRows = int64_t{1} << 24; // past this only 16 threads a row fit a launch
 
 void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float alpha,
                  const float* a, int64_t lda, const float* x, float beta, const float* y0,
@@ -418,7 +424,7 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
             const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
             gemv_n_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN), kWave * kWavesPerBlockN, 0,
                             s.stream>>>(a, lda, x, rows, cols, alpha, beta, y0, y);
-        } else if (rows >= kSharedRows && cols <= kNarrowCols) {
+        } else if (rows >= kSharedRows && (cols <= kNarrowCols || rows >= kManyRows)) {
             const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
             gemv_n_narrow_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN),
                                    kWave * kWavesPerBlockN, 0, s.stream>>>(
@@ -454,7 +460,9 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
         }
         mfr::check_launch("gemv_t_partial_kernel");
     }
-    gemv_t_finish_kernel<<<mfr::grid_blocks(cols, kWave), kWave * kFinishWaves, 0, s.stream>>>(
+    // At most 2^20 workgroups: a launch holds fewer than 2^32 threads.
+    gemv_t_finish_kernel<<<mfr::grid_blocks(cols, kWave, int64_t{1} << 20), kWave * kFinishWaves, 0,
+                           s.stream>>>(
         partial, chunks, cols, alpha, beta, y0, y);
     mfr::check_launch("gemv_t_finish_kernel");
 }
