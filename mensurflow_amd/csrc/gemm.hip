@@ -35,6 +35,7 @@
 //     own; the thin path (thin_kernel.hpp) takes products with at most 8 output columns or rows.
 #include "gemm_kernel.hpp"
 #include "panel_kernel.hpp"
+#include "regs_reach.hpp"
 #include "split.hpp"
 #include "thin_kernel.hpp"
 
@@ -385,8 +386,7 @@ bool split_takes(int tile, int64_t k) {
 // `blocks` workgroups of `tile` on the split kernel.
 void launch_split(int tile, const GemmParams& q, bool ak, bool bk, unsigned blocks, int cus,
                   hipStream_t stream) {
-    constexpr int64_t kFarLines = int64_t{1} << 26; // the register form's 32-bit offsets
-    const bool near = (ak || q.a_cs < kFarLines) && (bk || q.b_rs < kFarLines);
+    const bool near = (ak || regs_reach(q.a_cs)) && (bk || regs_reach(q.b_rs));
     switch (tile) {
     case MFR_TILE_256x256: launch_split_256x256(q, ak, bk, blocks, stream); break;
     case MFR_TILE_128x64: launch_split_128x64(q, ak, bk, blocks, stream); break;

@@ -10,7 +10,7 @@ void launch_split_256x256(const GemmParams& p, bool ak, bool bk, unsigned blocks
 void launch_split_128x128(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
 void launch_split_128x64(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
 void launch_split_64x128(const GemmParams& p, bool ak, bool bk, unsigned blocks, hipStream_t s);
-// No LDS in the depth loop; M/N-major lines less than 2^26 floats apart.
+// No LDS in the depth loop; M/N-major lines as regs_reach (regs_reach.hpp) allows.
 void launch_split_regs_64x64(const GemmParams& p, bool ak, bool bk, unsigned blocks,
                              hipStream_t s);
 // Likewise, on 64x64 tiles of which at most 32 rows are inside the matrix.

@@ -10,6 +10,7 @@
 // tiles, regions and splits around it.
 #pragma once
 
+#include "regs_reach.hpp"
 #include "split_parts.hpp"
 
 namespace mfr::gemm {
@@ -552,7 +553,7 @@ template <int F, bool KMAJ, int SETS = 1> struct StepLoader {
             if constexpr (KMAJ) {
                 at[f] = base + row * row_stride + 16 * first_step + 8 * half;
             } else {
-                offset[f] = static_cast<uint32_t>(8 * half * k_stride + row);
+                offset[f] = step_offset(k_stride, half, row);
             }
         }
     }

@@ -43,3 +43,9 @@ def test_device_gelu_arithmetic_every_61st_float():
     the reciprocal instruction. `gelu_exhaustive_test --stride 1` covers all 2^32 (about 90 s on
     8 threads; it passes as well)."""
     run("gelu_exhaustive_test", "--stride", "61")
+
+
+def test_gemm_register_form_reach():
+    """Every depth line stride the GEMM's register form is dispatched with (regs_reach) is one its
+    32-bit offsets hold: none that runs backwards or past 2^31 bytes within a step."""
+    run("gemm_reach_test")

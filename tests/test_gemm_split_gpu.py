@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import mensurflow_amd as mf
+from helpers import quarter_matrix
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +123,28 @@ def test_no_larger_error_than_fp32_chains(stream):
                           mf.DeviceArray.from_numpy(b, stream), tile=tile, splits=1).numpy()
             rel = np.linalg.norm(got - want) / np.linalg.norm(want)
             assert rel <= np.sqrt(k) * 2.0**-24 * 0.3, (k, tile, rel)
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 256, 256), (20, 250, 500), (200, 250, 71), (130, 70, 40)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_lines_that_run_backwards(stream, m, n, k, ta, tb):
+    """Operands whose lines lie a negative stride apart (the descriptor takes any element strides):
+    quarter integers, so the product is exact on AUTO and on every tile."""
+    a, b = quarter_matrix(m, k, 1), quarter_matrix(k, n, 2)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    # Stored along k or along m (n), the lines in reverse order.
+    a_d = mf.DeviceArray.from_numpy(np.ascontiguousarray((a.T if ta else a)[::-1]), stream)
+    b_d = mf.DeviceArray.from_numpy(np.ascontiguousarray((b.T if tb else b)[::-1]), stream)
+    c = mf.DeviceArray.empty((m, n), stream)
+    d = mf.GemmDesc()
+    d.m, d.n, d.k, d.alpha = m, n, k, 1.0
+    d.a = a_d.ptr + 4 * (a.size - (m if ta else k))
+    d.a_rs, d.a_cs = (1, -m) if ta else (-k, 1)
+    d.b = b_d.ptr + 4 * (b.size - (k if tb else n))
+    d.b_rs, d.b_cs = (1, -k) if tb else (-n, 1)
+    d.c, d.c_rs, d.stage = c.ptr, n, mf.abi.STAGE_NEVER
+    for tile in [mf.abi.TILE_AUTO] + TILES[1:]:  # the 256x256 tile refuses such lines
+        d.tile = tile
+        mf.fill(c, 7.0)
+        mf.sgemm(stream, d)
+        assert np.array_equal(c.numpy(), want), (tile, m, n, k, ta, tb)
