@@ -366,7 +366,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
     __shared__ uint4 tile_a1[LoadA::kPieces];
     __shared__ uint4 tile_b0[LoadB::kPieces];
     __shared__ uint4 tile_b1[LoadB::kPieces];
-    // The tanh gelu's exp table (see sgemm_direct_kernel), and what the end of the tile exchanges.
+    // The tanh gelu's exp table, and what the end of the tile exchanges.
     __shared__ double gelu_table[64];
     __shared__ float squares_of[WAVES_M * WAVES_N];
     __shared__ uint32_t unclear, smallest;
@@ -525,6 +525,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
             plain_blocks<FM, FN>(acc, a_base, b_base, p, kk, w.rows_a, w.rows_b, wave_m * WM,
                                  wave_n * WN, half, r32);
         }
+    } else {
+        lds_barrier(); // no depth, so no barrier yet: the gelu table is written
     }
     finish_tile<BM, BN, WM, WN, FM, FN>(acc, p, w, wave_m, wave_n, half, r32, gelu_table);
 }

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import mensurflow_amd as mf
-from helpers import quarter_matrix
+from helpers import quarter_matrix, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -148,3 +148,23 @@ def test_lines_that_run_backwards(stream, m, n, k, ta, tb):
         mf.fill(c, 7.0)
         mf.sgemm(stream, d)
         assert np.array_equal(c.numpy(), want), (tile, m, n, k, ta, tb)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_no_depth_gelu(stream, oracle, tile):
+    """A depth of 0 on a fixed tile: gelu(beta C0 + bias) bit for bit in every wavefront, the exp
+    table in LDS written before any of them reads it, right after a product that left other values
+    there."""
+    m, n = 300, 260
+    c0, bias = normal((m, n), 10), normal((n,), 11)
+    want = oracle.gelu(oracle.bias_add(np.float32(0.5) * c0, bias), approximate=True)
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    c0_d, bias_d = dev(c0), dev(bias)
+    a, b = mf.DeviceArray.empty((m, 0), stream), mf.DeviceArray.empty((0, n), stream)
+    other = dev(normal((512, 512), 12))
+    c = mf.DeviceArray.empty((m, n), stream)
+    for _ in range(5):
+        mf.gemm(other, other, tile=tile)
+        mf.fill(c, 7.0)
+        mf.gemm(a, b, c0=c0_d, beta=0.5, bias=bias_d, act=mf.ACT_GELU_TANH, tile=tile, out=c)
+        assert same_bits(c.numpy(), want)
