@@ -71,3 +71,16 @@ def test_nan_and_infinite_keys(stream):
         assert np.all(np.isnan(got[1])) and np.all(np.isfinite(got[[0, 2]]))
         want, scale = reference(q, k, v, np.ones((3, 2, lk), bool))
         assert np.all(np.abs(got - want)[[0, 2]] <= 1e-5 * np.sqrt(lk) * scale[[0, 2]])
+
+
+@pytest.mark.parametrize("lq,lk", [(1, 1), (1, 5000), (2, 300), (3, 2), (4, 4096)])
+def test_causal_reads_no_key_past_the_queries(stream, lq, lk):
+    """A long buffer whose keys and values past the queries were never written."""
+    rng = np.random.default_rng(lk)
+    q, k, v = (rng.standard_normal((2, 3, n, 64)).astype(np.float32) for n in (lq, lk, lk))
+    keep = np.tril(np.ones((lq, lk), bool))
+    want, scale = reference(q, k, v, keep)
+    k[..., lq:, :], v[..., lq:, :] = np.nan, np.inf
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    got = mf.attention_fused(dev(q), dev(k), dev(v), causal=True).numpy()
+    assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * scale)
