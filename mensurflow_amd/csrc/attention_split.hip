@@ -158,6 +158,9 @@ __device__ __forceinline__ void plain_queries(const AttnParams& p, const BlockWo
     const int64_t query = wq0 + r32;
     const float* q_row = p.q + work.off_q + (query < p.lq ? query : p.lq - 1) * p.q_rs;
     const float scale = p.scale * kLog2e;
+    // Causal: no key past the wavefront's own queries (k_end is the workgroup's), whose value might
+    // be infinite or NaN.
+    k_end = p.causal && k_end > wq0 + 32 ? wq0 + 32 : k_end;
     run = Running{};
 #pragma unroll
     for (int b = 0; b < DB; ++b) {

@@ -91,3 +91,21 @@ def test_mask_forms(stream, form):
             got = mf.attention_fused(dev(q), dev(k), dev(v), mask=mask).numpy()
             want, mag = reference(q, k, v, full)
             assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * mag), (form, d, lk)
+
+
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+def test_causal_rerun_reads_no_key_past_the_wavefront(stream, d):
+    """A value too small for its parts sends every wavefront through the fp32 matrix cores again;
+    the wavefronts whose queries come before a non-finite value stay finite."""
+    for batch, n in (((2,), 200), ((70, 4), 500)):  # 4 and 8 wavefronts a workgroup
+        rng = np.random.default_rng(d)
+        q, k, v = (rng.standard_normal(batch + (n, d)).astype(np.float32) for _ in range(3))
+        v[..., :64, 0] = 1e-37
+        keep = np.tril(np.ones((n, n), bool))
+        want, mag = reference(q, k, v, keep)
+        v[..., 64:, 1] = np.nan  # from the third wavefront's first query on
+        dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+        got = mf.attention_fused(dev(q), dev(k), dev(v), causal=True).numpy()
+        bound = 1e-5 * np.sqrt(n) * mag + n * 2.0**-149
+        assert np.all(np.abs(got - want)[..., :64, :] <= bound[..., :64, :]), (d, batch)
+        assert np.all(np.isnan(got[..., 96:, 1])), (d, batch)
