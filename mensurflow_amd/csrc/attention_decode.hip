@@ -259,9 +259,11 @@ void run_decode(mfr_stream& s, const AttnParams& given, int64_t d) {
         hold.lock();
         const size_t bytes =
             static_cast<size_t>(p.batch_count * p.lq * ranges * (d + 2)) * sizeof(float);
+        // Under stream capture one range: a graph would keep the workspace's address, which a later
+        // call may free to grow it, and its replays may run beside calls that use it.
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         mfr::check(hipStreamIsCapturing(s.stream, &capture), "hipStreamIsCapturing");
-        if (capture == hipStreamCaptureStatusNone || bytes <= s.workspace_bytes) {
+        if (capture == hipStreamCaptureStatusNone) {
             try {
                 parts = static_cast<float*>(s.reserve(bytes));
             } catch (const mfr::Error&) {

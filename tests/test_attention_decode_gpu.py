@@ -84,3 +84,46 @@ def test_causal_reads_no_key_past_the_queries(stream, lq, lk):
     dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
     got = mf.attention_fused(dev(q), dev(k), dev(v), causal=True).numpy()
     assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * scale)
+
+
+def test_captured_call_keeps_no_workspace():
+    """A captured call's graph is replayed after eager calls on the same stream have used and grown
+    the stream's workspace, and after the inputs changed."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library has loaded
+
+    def call(name, *args):
+        assert getattr(hip, name)(*args) == 0, name
+
+    heads, lk, d = 6, 4096, 64
+    rng = np.random.default_rng(7)
+    host = lambda n: rng.standard_normal((heads, n, d)).astype(np.float32)  # noqa: E731
+    with mf.Stream(0) as stream:
+        q, k, v = (mf.DeviceArray.from_numpy(host(n), stream) for n in (1, lk, lk))
+        out = mf.DeviceArray.empty((heads, 1, d), stream)
+
+        def check():
+            want, scale = reference(q.numpy(), k.numpy(), v.numpy(), np.ones((heads, 1, lk), bool))
+            assert np.all(np.abs(out.numpy() - want) <= 1e-5 * np.sqrt(lk) * scale)
+
+        mf.attention_fused(q, k, v, out=out)  # the workspace holds the ranges' results from here on
+        check()
+        handle = ctypes.c_void_p(stream.hip_stream())
+        graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+        thread_local = 1  # hipStreamCaptureModeThreadLocal
+        call("hipStreamBeginCapture", handle, ctypes.c_int(thread_local))
+        mf.attention_fused(q, k, v, out=out)
+        call("hipStreamEndCapture", handle, ctypes.byref(graph))
+        call("hipGraphInstantiate", ctypes.byref(run), graph, None, None, ctypes.c_size_t(0))
+        for size in (256, 4096, 16384):  # y = A^T x: partial sums, a larger workspace each time
+            a = mf.DeviceArray.from_numpy(rng.standard_normal((2048, size)).astype(np.float32), stream)
+            x = mf.DeviceArray.from_numpy(rng.standard_normal(2048).astype(np.float32), stream)
+            mf.sgemv(a, x, trans=True)
+            q.upload(host(1))
+            v.upload(host(lk))
+            mf.fill(out, 7.0)
+            call("hipGraphLaunch", run, handle)
+            check()
+        call("hipGraphExecDestroy", run)
+        call("hipGraphDestroy", graph)
