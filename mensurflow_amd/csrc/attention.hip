@@ -2,7 +2,7 @@
 // softmax(scale * q k^T, masked) v without writing the [.., lq, lk] scores to memory; the
 // reference composes the same op from a batched GEMM, where(), softmax and a second batched GEMM
 // (src/ops/attention.cpp:48-98). d = 32, 64, 96 and 128 run on the bf16 matrix cores
-// (attention_split.hip) and at most 4 queries in the decode form (attention_decode.hip); this file
+// (attention_split.hip) and 1 to 4 queries mostly in the decode form (attention_decode.hip); this file
 // holds the entry point and the fp32 matrix core kernel of d = 16, 48, 80 and 112.
 //
 // Design (a workgroup of 4 wavefronts of 32 queries; keys in blocks of BK):
@@ -409,7 +409,8 @@ void run_attention(mfr_stream& s, const mfr_attention_desc& d) {
     p.out = d.out;
     p.mask = d.mask;
     p.lq = d.lq;
-    p.lk = d.lk;
+    // Causal query i keeps keys 0 .. i: no form reads those past the last query.
+    p.lk = d.causal != 0 && d.lq < d.lk ? d.lq : d.lk;
     p.q_rs = d.q_rs;
     p.k_rs = d.k_rs;
     p.v_rs = d.v_rs;
@@ -429,7 +430,7 @@ void run_attention(mfr_stream& s, const mfr_attention_desc& d) {
     p.causal = d.causal != 0;
     p.scale = d.scale != 0.0f ? d.scale
                               : static_cast<float>(1.0 / std::sqrt(static_cast<double>(d.d)));
-    if (d.lq <= mfr::attn::kDecodeMaxQueries && d.lk > 0) {
+    if (mfr::attn::decode_takes(p.lq, p.lk, d.d, batch_count, s.compute_units)) {
         mfr::attn::run_decode(s, p, d.d);
         return;
     }

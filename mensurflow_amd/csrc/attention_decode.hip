@@ -237,13 +237,8 @@ void launch_queries(const AttnParams& p, int d, int ranges, int64_t range, float
 
 namespace mfr::attn {
 
-void run_decode(mfr_stream& s, const AttnParams& given, int64_t d) {
+void run_decode(mfr_stream& s, const AttnParams& p, int64_t d) {
     static_assert(kDecodeMaxQueries == 4, "launch_queries covers every count");
-    AttnParams p = given;
-    if (p.causal != 0) {
-        // Query i keeps keys 0 .. i: those past the last query are not read.
-        p.lk = std::min(p.lk, p.lq);
-    }
     // Ranges of at least 256 keys, for about 4 workgroups per CU; one range needs no workspace.
     constexpr int64_t kLeastKeys = 256;
     constexpr int64_t kMostRanges = 64;

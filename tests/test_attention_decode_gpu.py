@@ -73,17 +73,27 @@ def test_nan_and_infinite_keys(stream):
         assert np.all(np.abs(got - want)[[0, 2]] <= 1e-5 * np.sqrt(lk) * scale[[0, 2]])
 
 
-@pytest.mark.parametrize("lq,lk", [(1, 1), (1, 5000), (2, 300), (3, 2), (4, 4096)])
-def test_causal_reads_no_key_past_the_queries(stream, lq, lk):
+@pytest.mark.parametrize("lq,lk", [(1, 1), (1, 5000), (2, 300), (3, 2), (4, 4096), (40, 50)])
+@pytest.mark.parametrize("d", [32, 64, 80])
+def test_causal_reads_no_key_past_the_queries(stream, d, lq, lk):
     """A long buffer whose keys and values past the queries were never written."""
     rng = np.random.default_rng(lk)
-    q, k, v = (rng.standard_normal((2, 3, n, 64)).astype(np.float32) for n in (lq, lk, lk))
+    q, k, v = (rng.standard_normal((2, 3, n, d)).astype(np.float32) for n in (lq, lk, lk))
     keep = np.tril(np.ones((lq, lk), bool))
     want, scale = reference(q, k, v, keep)
     k[..., lq:, :], v[..., lq:, :] = np.nan, np.inf
     dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
     got = mf.attention_fused(dev(q), dev(k), dev(v), causal=True).numpy()
     assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * scale)
+
+
+@pytest.mark.parametrize("d,lq,lk", [(16, 2, 256), (32, 2, 128), (64, 3, 128), (32, 4, 256),
+                                     (32, 4, 2048), (128, 4, 64), (48, 4, 256), (16, 3, 1024)])
+def test_form_lines(stream, d, lq, lk):
+    """Both sides of the lines between the decode form and the tile kernels, in keys and heads."""
+    for heads in (127, 128, 129, 257):
+        for keys in (lk - 1, lk):
+            check(stream, (heads,), lq, keys, d, seed=heads + keys)
 
 
 def test_captured_call_keeps_no_workspace():
