@@ -109,3 +109,17 @@ def test_causal_rerun_reads_no_key_past_the_wavefront(stream, d):
         bound = 1e-5 * np.sqrt(n) * mag + n * 2.0**-149
         assert np.all(np.abs(got - want)[..., :64, :] <= bound[..., :64, :]), (d, batch)
         assert np.all(np.isnan(got[..., 96:, 1])), (d, batch)
+
+
+@pytest.mark.parametrize("d", [64, 96])
+@pytest.mark.parametrize("lq,lk", [(5, 512), (128, 512), (128, 513), (129, 100), (33, 33)])
+def test_workgroup_sizes(stream, d, lq, lk):
+    """Workgroups of 4 and of 8 wavefronts, on enough heads for either."""
+    rng = np.random.default_rng(lq + lk)
+    q, k, v = (rng.standard_normal((520, n, d)).astype(np.float32) for n in (lq, lk, lk))
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    for causal in (False, True):
+        keep = np.tril(np.ones((lq, lk), bool)) if causal else np.ones((lq, lk), bool)
+        got = mf.attention_fused(dev(q), dev(k), dev(v), causal=causal).numpy()
+        want, mag = reference(q[::40], k[::40], v[::40], keep)
+        assert np.all(np.abs(got[::40] - want) <= 1e-5 * np.sqrt(lk) * mag), causal
