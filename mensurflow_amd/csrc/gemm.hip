@@ -106,10 +106,20 @@ int splits_for(int64_t k, int64_t per) { return static_cast<int>((k + per - 1) /
 // form (sgemm_split_regs_kernel): every CU has at most one workgroup, and either more than half
 // of them have one or the depth is short; AUTO splits a longer depth over the idle CUs. 1024^3
 // 24.8 -> 20.7 us.
-constexpr int64_t kFewRows = 32; // at most this many rows run its 32x64 form, split or not
+constexpr int64_t kFewRows = 32; // at most this many rows may run its 32x64 form, split or not
 
 bool regs_form(int64_t count, int64_t k, int cus) {
     return count <= cus && (2 * count > cus || k <= 512);
+}
+
+// Whether a product of at most kFewRows rows runs `count` 64x64 tiles (every range counted) of depth
+// k in the 32x64 register form. With several tiles per CU and a short depth its 8 wavefronts have
+// little to share and the exchange counts: 4096 x [32 x 72 x 64] 76 us against 46 in the LDS form,
+// depth 128 69 against 52, 256 124 against 100; at a depth of 512 and more, or read along n on at
+// most 2 per CU, it is even or ahead (300 x [32 x 256 x 64] along n 16 %, 1024 x [32 x 1024 x 64]
+// 8 %), as it is for a split product's ranges, whose operand comes from HBM once.
+bool few_rows_form(int64_t count, int64_t k, int splits, bool bk, int cus) {
+    return count <= cus || splits > 1 || k >= 512 || (!bk && k >= 128 && count <= 2 * cus);
 }
 
 // Modelled time (us) of tile t with `splits` depth ranges of `per` each: the launch, the busiest
@@ -118,13 +128,15 @@ bool regs_form(int64_t count, int64_t k, int cus) {
 // 200^3 to 4096^3. On each shape the model's pick measures within 3 % of the
 // best point, 0.2 % on average.
 double modelled_us(int t, int64_t m, int64_t n, int64_t k, int64_t batch, int cus, int splits,
-                   int64_t per, bool c0) {
+                   int64_t per, bool c0, bool bk) {
     const TileInfo& info = kTiles[t];
     const int64_t count = tile_count(t, m, n, batch) * splits;
     const int64_t per_cu = (count + cus - 1) / cus;
     const int64_t resident = per_cu < info.occupancy ? per_cu : info.occupancy;
-    const bool regs = t == MFR_TILE_64x64 &&
-                      (m <= kFewRows || (splits == 1 && regs_form(count, k, cus)));
+    const bool regs =
+        t == MFR_TILE_64x64 &&
+        ((m <= kFewRows && few_rows_form(count, splits > 1 ? per : k, splits, bk, cus)) ||
+         (splits == 1 && regs_form(count, k, cus)));
     const double depth = static_cast<double>(splits > 1 ? per : k);
     const double tile_us = regs ? kRegsDepthUs * depth + kRegsFixedUs
                                 : info.depth_us[resident - 1] * depth +
@@ -238,7 +250,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int cus,
         const int64_t a = tile_count(MFR_TILE_128x64, m, n, batch) * 128 * 64;
         const int64_t b = tile_count(MFR_TILE_64x128, m, n, batch) * 64 * 128;
         best.tile = b < a ? MFR_TILE_64x128 : MFR_TILE_128x64;
-        best.us = modelled_us(best.tile, m, n, k, batch, cus, 1, k, c0);
+        best.us = modelled_us(best.tile, m, n, k, batch, cus, 1, k, c0, bk);
     } else {
         double best_us = 1e300;
         for (int t = 1; t < MFR_TILE_THIN; ++t) {
@@ -248,7 +260,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int cus,
             }
             if (fixed_splits > 0) {
                 // Only the tile is open.
-                const double us = modelled_us(t, m, n, k, batch, cus, best.splits, best.per, c0);
+                const double us = modelled_us(t, m, n, k, batch, cus, best.splits, best.per, c0, bk);
                 if (us < best_us) {
                     best_us = us;
                     best.tile = t;
@@ -269,7 +281,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int cus,
                      4.0 * splits * static_cast<double>(m) * n * batch > kMaxPartialBytes)) {
                     break;
                 }
-                const double us = modelled_us(t, m, n, k, batch, cus, splits, per, c0);
+                const double us = modelled_us(t, m, n, k, batch, cus, splits, per, c0, bk);
                 if (us < best_us) {
                     best_us = us;
                     best.tile = t;
@@ -393,7 +405,8 @@ void launch_split(int tile, const GemmParams& q, bool ak, bool bk, unsigned bloc
     case MFR_TILE_64x128: launch_split_64x128(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x64:
         // (512 threads a workgroup, fewer than 2^32 in a launch.)
-        if (q.m <= kFewRows && near && blocks < (1u << 23)) {
+        if (q.m <= kFewRows && near && blocks < (1u << 23) &&
+            few_rows_form(blocks, q.k_per_split, q.splits, bk, cus)) {
             launch_split_regs_32x64(q, ak, bk, blocks, stream);
         } else if (q.splits == 1 && regs_form(blocks, q.k, cus) && near) {
             launch_split_regs_64x64(q, ak, bk, blocks, stream);

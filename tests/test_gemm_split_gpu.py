@@ -168,3 +168,20 @@ def test_no_depth_gelu(stream, oracle, tile):
         mf.fill(c, 7.0)
         mf.gemm(a, b, c0=c0_d, beta=0.5, bias=bias_d, act=mf.ACT_GELU_TANH, tile=tile, out=c)
         assert same_bits(c.numpy(), want)
+
+
+@pytest.mark.parametrize("batch", [256, 257, 513])
+@pytest.mark.parametrize("k", [72, 127, 128, 511, 512])
+def test_few_rows_batched_exact(stream, batch, k):
+    """At most 32 rows and one 64-column tile a matrix: both sides of the register form's lines, in
+    tiles and in depth, exact on quarter integers."""
+    m, n = 19, 61
+    a = quarter_matrix(batch * m, k, 1).reshape(batch, m, k)
+    b = quarter_matrix(batch * k, n, 2).reshape(batch, k, n)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    a_d = mf.DeviceArray.from_numpy(a, stream)
+    c = mf.DeviceArray.empty((batch, m, n), stream)
+    for tb in (False, True):
+        b_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(np.swapaxes(b, 1, 2) if tb else b), stream)
+        mf.gemm_batched(a_d, b_d.transpose(-2, -1) if tb else b_d, c)
+        assert np.array_equal(c.numpy(), want), tb
