@@ -39,7 +39,7 @@ def test_softmax_and_argmax(stream, oracle, width):
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 2), (1, 4099), (64, 5), (2047, 257),
-                                       (2048, 1024), (2050, 1023), (8191, 300), (8200, 64),
+                                       (2048, 1024), (2050, 1023), (8191, 300), (4001, 512), (8200, 64),
                                        (300, 16383), (4093, 1023), (16, 20000)])
 def test_gemv_exact(stream, rows, cols):
     """Quarter integers: exact sums, so exact results, N and T, on whole and offset storage."""
@@ -58,3 +58,13 @@ def test_gemv_exact(stream, rows, cols):
                          y0=mf.DeviceArray.from_numpy(y0, stream), trans=trans).numpy()
             want = 2.0 * ((a64.T if trans else a64) @ x.astype(np.float64)) + 0.5 * y0
             assert same_bits(y, want.astype(np.float32)), (rows, cols, trans, offset)
+
+
+@pytest.mark.parametrize("rows,width", [(4096, 1024), (4096, 1025), (4097, 1025),
+                                        (4097, 3072), (4097, 3073)])
+def test_argmax_many_rows(stream, rows, width):
+    """Both sides of the line between a wavefront and a workgroup a row, ties to the lower index."""
+    x = np.random.default_rng(rows).integers(-500, 500, (rows, width)).astype(np.float32)
+    x[::7, width - 1] = np.nan
+    got = mf.argmax(mf.DeviceArray.from_numpy(x, stream)).numpy()
+    assert np.array_equal(got, np.argmax(np.where(np.isnan(x), np.inf, x), axis=1))
