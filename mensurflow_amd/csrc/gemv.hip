@@ -420,7 +420,7 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
     const bool vec4 = mfr::aligned16(a) && lda % 4 == 0 && cols % 4 == 0 &&
                       (!trans ? mfr::aligned16(x) : true);
     if (!trans) {
-        if (vec4 && rows >= kStreamRows) {
+        if (vec4 && (rows >= kStreamRows || (rows >= kSharedRows && cols <= kNarrowCols))) {
             const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
             gemv_n_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN), kWave * kWavesPerBlockN, 0,
                             s.stream>>>(a, lda, x, rows, cols, alpha, beta, y0, y);
