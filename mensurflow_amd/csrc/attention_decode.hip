@@ -79,16 +79,15 @@ __global__ __launch_bounds__(kWaves * 64) void attention_decode_kernel(AttnParam
     const int64_t first = index * range;
     const int64_t end = first + range < p.lk ? first + range : p.lk;
 
-    // The queries times scale log2 e, so scores are base-2 exponents.
+    // Scores are scaled after their products (as the tile kernels' are where it matters), so that
+    // only they can overflow, and are base-2 exponents.
     float4 q[QN], acc[QN];
     float top[QN], sum[QN];
-    const float scale = p.scale * kLog2e;
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
         q[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (live && i < p.lq) {
-            const float4 v = *reinterpret_cast<const float4*>(p.q + off_q + i * p.q_rs + depth);
-            q[i] = make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
+            q[i] = *reinterpret_cast<const float4*>(p.q + off_q + i * p.q_rs + depth);
         }
         acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         top[i] = -INFINITY;
@@ -119,7 +118,7 @@ __global__ __launch_bounds__(kWaves * 64) void attention_decode_kernel(AttnParam
                 s = fmaf(q[i].y, k[u].y, s);
                 s = fmaf(q[i].z, k[u].z, s);
                 s = fmaf(q[i].w, k[u].w, s);
-                s = group_sum<G>(s);
+                s = p.scale * group_sum<G>(s) * kLog2e;
                 bool keep = key < end && i < p.lq && (p.causal == 0 || key <= i);
                 if (keep && p.mask != nullptr) {
                     keep = p.mask[off_m + i * p.mask_rs + key * p.mask_cs] != 0;

@@ -87,6 +87,18 @@ def test_causal_reads_no_key_past_the_queries(stream, d, lq, lk):
     assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * scale)
 
 
+@pytest.mark.parametrize("lk", [300, 5000])
+def test_scale_applies_to_the_scores(stream, lk):
+    """scale q overflows where scale (q k) is ordinary."""
+    rng = np.random.default_rng(lk)
+    q, k, v = (rng.standard_normal((2, 3, n, 64)).astype(np.float32) for n in (1, lk, lk))
+    q, k = q * np.float32(2.0**112), k * np.float32(2.0**-132)
+    want, scale = reference(q.astype(np.float64) * 2.0**20, k, v, np.ones((1, lk), bool))
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    got = mf.attention_fused(dev(q), dev(k), dev(v), scale=2.0**20 / 8).numpy()
+    assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(lk) * scale)
+
+
 @pytest.mark.parametrize("d,lq,lk", [(16, 2, 256), (32, 2, 128), (64, 3, 128), (32, 4, 256),
                                      (32, 4, 2048), (128, 4, 64), (48, 4, 256), (16, 3, 1024)])
 def test_form_lines(stream, d, lq, lk):
