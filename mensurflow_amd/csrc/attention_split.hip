@@ -146,9 +146,25 @@ __device__ __forceinline__ void softmax_step(floatx16 (&s)[SUB], floatx16 (&o)[D
     }
 }
 
-// The wavefront's queries on the fp32 matrix cores, straight from global memory: what it runs again
-// when a result is not finite (an infinite or NaN operand has NaN parts whatever it meets) or the
-// values hold elements too small for their parts.
+// ---- where the part products do not stand for the fp32 products --------------------------------
+//
+// A wavefront runs its queries again on the fp32 matrix cores (plain_queries) when
+//   - a result is not finite: an infinite or NaN operand has NaN parts whatever it meets, one above
+//     the largest bf16 (or a query that its scale takes there) infinite ones;
+//   - its scores may have lost something: parts and part products under 2^-126 count as lost, so a
+//     score misses at most 2^-126 (sqrt(d) (|q| + |k|) + 6 d), an absolute error of its base-2
+//     exponent. With the squares of the workgroup's keys and of the lane's query (both as cut)
+//     summing to less than 2^126, that is under 2^-58;
+//   - an output may have: its terms lose at most 2^-126 (6 + |v|) a key. 2^26 times as much, with a
+//     little room (the bound below, the sum of the squares for the largest value), stays under the
+//     output's own rounding. A smaller output is run again, but one of exactly 0 only where values
+//     under 2^-49 were met: without them it stands for weights below 2^-73, 2^-122 in all.
+// So zero values, and a few tiny ones among others, cost nothing.
+constexpr uint32_t kSmallestValue = (127u - 49u) << 23;
+constexpr float kMostSquares = 0x1p126f;
+
+// The wavefront's queries on the fp32 matrix cores, straight from global memory, scaled after their
+// products as the kernel of attention.hip scales them.
 template <int D, MaskForm MASK>
 __device__ __forceinline__ void plain_queries(const AttnParams& p, const BlockWork& work,
                                               const uint8_t* mask_row, int64_t wq0, int64_t k_end,
@@ -157,7 +173,6 @@ __device__ __forceinline__ void plain_queries(const AttnParams& p, const BlockWo
     constexpr int DB = D / 32;
     const int64_t query = wq0 + r32;
     const float* q_row = p.q + work.off_q + (query < p.lq ? query : p.lq - 1) * p.q_rs;
-    const float scale = p.scale * kLog2e;
     // Causal: no key past the wavefront's own queries (k_end is the workgroup's), whose value might
     // be infinite or NaN.
     k_end = p.causal && k_end > wq0 + 32 ? wq0 + 32 : k_end;
@@ -180,8 +195,12 @@ __device__ __forceinline__ void plain_queries(const AttnParams& p, const BlockWo
         const float* k_row = p.k + work.off_k + key * p.k_rs;
 #pragma unroll 2
         for (int depth = 0; depth < D; depth += 2) {
-            s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(k_row[depth + half],
-                                                        q_row[depth + half] * scale, s[0], 0, 0, 0);
+            s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(k_row[depth + half], q_row[depth + half],
+                                                        s[0], 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            s[0][e] = p.scale * s[0][e] * kLog2e;
         }
         uint32_t bits = 0;
         if constexpr (MASK != kNoMask) {
@@ -223,6 +242,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
     __shared__ uint4 k_tile0[kPiecesK], k_tile1[kPiecesK];
     __shared__ uint4 v_tile0[kPiecesV], v_tile1[kPiecesV];
     __shared__ uint32_t smallest;
+    __shared__ float k_squares_of[WAVES], v_squares_of[WAVES];
     if (threadIdx.x == 0) {
         smallest = 0xffffffffu;
     }
@@ -243,7 +263,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
 
     // q times scale log2 e, cut: depth 16 step + 8 half + j of the lane's query.
     bf16x8 qf[STEPS][3];
-    float unused = 0.0f;
+    float q_squares = 0.0f, k_squares = 0.0f, v_squares = 0.0f;
     {
         const float scale = p.scale * kLog2e;
         const float* q_row = p.q + work.off_q + (query < p.lq ? query : p.lq - 1) * p.q_rs;
@@ -254,7 +274,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
             const float x[8] = {lo.x * scale, lo.y * scale, lo.z * scale, lo.w * scale,
                                 hi.x * scale, hi.y * scale, hi.z * scale, hi.w * scale};
             uint32_t part[3][4];
-            cut_eight(x, part, unused);
+            cut_eight(x, part, q_squares);
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
                 qf[st][i] = __builtin_bit_cast(
@@ -315,7 +335,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
                 break;
             }
             uint32_t part[3][4];
-            cut_eight(k_reg[i], part, unused);
+            cut_eight(k_reg[i], part, k_squares);
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 k_tile[(q * kGroupsK + u % kGroupsK) * kPitchK + u / kGroupsK] =
@@ -325,7 +345,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
             for (int j = 0; j < 8; ++j) {
                 least = min(least, (__float_as_uint(v_reg[i][j]) & 0x7fffffffu) - 1);
             }
-            cut_eight(v_reg[i], part, unused);
+            cut_eight(v_reg[i], part, v_squares);
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 v_tile[(q * kGroupsV + u / D) * kPitchV + u % D] =
@@ -404,6 +424,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
                         w[j] = s[t / 2][8 * (t % 2) + j];
                     }
                     uint32_t part[3][4];
+                    float unused = 0.0f;
                     cut_eight(w, part, unused);
 #pragma unroll
                     for (int q = 0; q < 3; ++q) {
@@ -445,26 +466,53 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
         }
     }
 
-    // Values under 2^-100 (not zero) have parts under 2^-126.
-    constexpr uint32_t kSmallestValue = (127u - 100u) << 23;
     if (__any(least < kSmallestValue - 1)) {
         atomicMin(&smallest, least);
+    }
+    k_squares = mfr::dev::butterfly_sum(k_squares);
+    v_squares = mfr::dev::butterfly_sum(v_squares);
+    if (lane == 0) {
+        k_squares_of[wave] = k_squares;
+        v_squares_of[wave] = v_squares;
     }
     lds_barrier();
     if (!wave_live) {
         return;
     }
+    k_squares = v_squares = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        k_squares += k_squares_of[w];
+        v_squares += v_squares_of[w];
+    }
     float total = sum_halves(run.sum);
     float zero = total * 0.0f; // NaN once a result is not finite
+    float least_out = __builtin_inff();
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             zero = fmaf(oacc[b][e], 0.0f, zero);
+            least_out = fminf(least_out, __builtin_fabsf(oacc[b][e]));
         }
     }
-    const bool again = !__all(zero == 0.0f) || smallest < kSmallestValue - 1;
-    if (__builtin_amdgcn_readfirstlane(again) != 0) {
+    const float bound =
+        static_cast<float>(k_end) * 0x1p-97f * (8.0f + fminf(sqrtf(v_squares), 0x1p127f));
+    bool again = zero != 0.0f || !(q_squares < kMostSquares) || !(k_squares < kMostSquares);
+    if (__any(least_out < bound) && !__any(again)) {
+        // The least output that is not 0, as bits - 1 (0 wraps past all), against the bound.
+        uint32_t nonzero = 0xffffffffu;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                nonzero = min(nonzero, (__float_as_uint(oacc[b][e]) & 0x7fffffffu) - 1);
+            }
+        }
+        again = nonzero < __float_as_uint(bound) - 1 ||
+                (least_out == 0.0f && smallest < kSmallestValue - 1);
+    }
+    if (__any(again)) {
         plain_queries<D, MASK>(p, work, mask_row, wq0, k_end, half, r32, oacc, run);
         total = sum_halves(run.sum);
     }

@@ -9,9 +9,10 @@ import mensurflow_amd as mf
 pytestmark = pytest.mark.gpu
 
 
-def reference(q, k, v, keep):
+def reference(q, k, v, keep, scale=None):
     with np.errstate(all="ignore"):
-        s = q.astype(np.float64) @ np.swapaxes(k.astype(np.float64), -1, -2) / np.sqrt(q.shape[-1])
+        s = q.astype(np.float64) @ np.swapaxes(k.astype(np.float64), -1, -2)
+        s = s * (1 / np.sqrt(q.shape[-1]) if scale is None else scale)
         s = np.where(keep, s, -np.inf)
         top = np.max(s, axis=-1, keepdims=True)
         p = np.exp(s - np.where(top == -np.inf, 0.0, top))
@@ -28,7 +29,9 @@ def reference(q, k, v, keep):
 
 @pytest.mark.parametrize("d", [32, 64, 96, 128])
 @pytest.mark.parametrize("case", ["value inf", "value nan", "key -inf", "key nan", "huge value",
-                                  "tiny values", "huge scores"])
+                                  "tiny values", "huge scores", "tiny keys", "tiny queries",
+                                  "huge scale", "small values", "smaller values", "one tiny value",
+                                  "tiny column", "values of the least weights"])
 def test_extreme_operands(stream, d, case):
     for batch, lq, lk, causal in (((2,), 70, 150, False), ((2,), 260, 260, True),
                                   ((70, 4), 300, 64, False)):
@@ -54,10 +57,31 @@ def test_extreme_operands(stream, d, case):
         elif case == "huge scores":
             q *= np.float32(1e18)
             k *= np.float32(1e18)
+        elif case in ("tiny keys", "tiny queries"):  # ordinary scores of parts under 2^-126
+            q, k = q * np.float32(1e36), k * np.float32(1e-36)
+            if case == "tiny queries":
+                q, k = q * np.float32(1e-36) * np.float32(1e-36), k * np.float32(1e36) * np.float32(1e36)
+        elif case == "huge scale":  # scale q overflows, scale (q k) does not
+            q, k = q * np.float32(1e35), k * np.float32(1e-39)
+        elif case == "small values":
+            v *= np.float32(2.0**-60)
+        elif case == "smaller values":
+            v *= np.float32(2.0**-95)
+        elif case == "one tiny value":
+            v[one + (0, 0)] = 1e-37
+        elif case == "tiny column":
+            v[..., 1] *= np.float32(1e-33)
+        elif case == "values of the least weights":  # the likeliest keys' values are 0
+            # Scores up to 25 in size: their rounding moves a weight by 25 * 2^-22, 6e-6 of it.
+            k *= np.float32(4.0)
+            top = np.argmax(q @ np.swapaxes(k, -1, -2), axis=-1)
+            for idx in np.ndindex(batch):
+                v[idx][np.unique(top[idx]), 2] = 0.0
+        scale = 1e4 if case == "huge scale" else None
         keep = np.tril(np.ones((lq, lk), bool)) if causal else np.ones((lq, lk), bool)
         dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
-        got = mf.attention_fused(dev(q), dev(k), dev(v), causal=causal).numpy()
-        want, mag = reference(q, k, v, keep)
+        got = mf.attention_fused(dev(q), dev(k), dev(v), causal=causal, scale=scale or 0.0).numpy()
+        want, mag = reference(q, k, v, keep, scale)
         what = (case, d, batch, lq, lk)
         assert np.array_equal(np.isnan(got), np.isnan(want)), what
         ok = np.isfinite(want)
@@ -123,3 +147,16 @@ def test_workgroup_sizes(stream, d, lq, lk):
         got = mf.attention_fused(dev(q), dev(k), dev(v), causal=causal).numpy()
         want, mag = reference(q[::40], k[::40], v[::40], keep)
         assert np.all(np.abs(got[::40] - want) <= 1e-5 * np.sqrt(lk) * mag), causal
+
+
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("lq,lk", [(150, 1024), (520, 333)])
+def test_every_part_counts(stream, d, lq, lk):
+    """The 2-norm error on normal operands is the fp32 sums' own (2.8e-7 to 5.3e-7 measured): a lost
+    part of q, k, v or the weights, 2^-17 of it, would be 10 times the bound."""
+    rng = np.random.default_rng(d)
+    q, k, v = (rng.standard_normal((3, n, d)).astype(np.float32) for n in (lq, lk, lk))
+    dev = lambda x: mf.DeviceArray.from_numpy(x, stream)  # noqa: E731
+    got = mf.attention_fused(dev(q), dev(k), dev(v)).numpy()
+    want, _ = reference(q, k, v, np.ones((lq, lk), bool))
+    assert np.linalg.norm(got - want) <= 8e-7 * np.linalg.norm(want)
