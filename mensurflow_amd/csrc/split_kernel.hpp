@@ -458,6 +458,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
         }
         lds_barrier();
     };
+    if (slices == 0) {
+        lds_barrier(); // no depth, so no other: the gelu table is written
+    }
     if (slices > 0) {
         load(0);
         la.cut_and_store(tile_a0, squares);
@@ -525,8 +528,6 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
             plain_blocks<FM, FN>(acc, a_base, b_base, p, kk, w.rows_a, w.rows_b, wave_m * WM,
                                  wave_n * WN, half, r32);
         }
-    } else {
-        lds_barrier(); // no depth, so no barrier yet: the gelu table is written
     }
     finish_tile<BM, BN, WM, WN, FM, FN>(acc, p, w, wave_m, wave_n, half, r32, gelu_table);
 }
