@@ -24,18 +24,25 @@ namespace mfr::gemm {
 //   - they are small next to what can have been lost: at most 2^-126 in each part of an element,
 //     times the largest element it meets, and in each of the six part products, over the depth.
 //     2^26 times as much would stay under the sums' own rounding.
-// A wavefront whose sums are finite and clear of that bound is done (the bound takes the sum of
-// the squares of the tile's elements for their largest: 2^-85 for a few thousand normal values).
+// A wavefront whose sums are finite and clear of that bound is done (sums_bound: 2^-74 for 4096
+// depths of a million normal values).
 // Where a few sums are not clear (a sum that happens to be 0), the wavefront reads their rows and
 // columns again for their smallest nonzero magnitude; with more of them (padding rows), the
 // workgroup reads its operands again. A wavefront runs its blocks on the fp32 matrix cores
 // (plain_blocks) where that is under 2^-49 or a sum is not finite. So zeros cost a second read
-// only where sums are zero too, and a few tiny elements among others (softmax weights) nothing.
+// only where sums are zero too (1024^3 with zero rows in A 20 -> 31 us, 2048^3 94 -> 121, 4096^3 570 ->
+// 680), and a few tiny elements among others (softmax weights) nothing.
 // (Keeping the least magnitude beside the squares instead cost 7 % at 4096^3: every operation
 // per element cut adds to a loop that is bound by issue and by power.)
 
 constexpr uint32_t kSmallest = (127u - 49u) << 23; // 2^-49
 constexpr int kFewLines = 4;
+
+// What a sum of kk products has to reach to be clear: `squares` is the sum of the squares of the
+// tile's elements, whose root is at least the largest.
+__device__ __forceinline__ float sums_bound(float squares, int64_t kk) {
+    return 2.0f * (1.0f + sqrtf(squares)) * static_cast<float>(kk) * 0x1p-97f;
+}
 
 enum class Sums { kClear, kUnclear, kNotFinite };
 
@@ -281,10 +288,34 @@ template <int ROWS, int KT, bool KMAJ, int THREADS> struct SplitLoader {
     }
 };
 
+// Eight depths of a row, from `at` on.
+template <bool KMAJ>
+__device__ __forceinline__ void load_eight(float (&v)[8], const float* at, int64_t stride) {
+    if constexpr (KMAJ) {
+        typedef native4 __attribute__((aligned(4))) loose4;
+        const native4 lo = *reinterpret_cast<const loose4*>(at);
+        const native4 hi = *reinterpret_cast<const loose4*>(at + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = lo[e];
+            v[4 + e] = hi[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[e] = *at;
+            at += stride;
+        }
+    }
+}
+
 // The wavefront's blocks on the fp32 matrix cores, straight from global memory: what a tile runs
 // again where the part products do not stand for its products. Rows past the matrix repeat
-// its last row.
-template <int FM, int FN>
+// its last row. Lanes 0-31 take eight depths of their rows at a time, lanes 32-63 the next eight
+// (2048^3 with one infinite element 570 -> 247 us against one depth each, 1024^3 121 -> 56); not
+// for the 256x256 tile's 8 blocks, where the compiler then orders the main loop's loads and cuts
+// another way (4096^3 608 -> 622 us, the MLP 188 -> 197).
+template <int FM, int FN, bool AK, bool BK>
 __device__ __forceinline__ void plain_blocks(floatx16 (&acc)[FM][FN], const float* a_base,
                                              const float* b_base, const GemmParams& p, int64_t kk,
                                              int rows_a, int rows_b, int row0, int col0, int half,
@@ -311,8 +342,35 @@ __device__ __forceinline__ void plain_blocks(floatx16 (&acc)[FM][FN], const floa
             }
         }
     }
+    int64_t k = 0;
+    if constexpr (FM * FN <= 2) {
 #pragma unroll 1
-    for (int64_t k = 0; k < kk; k += 2) {
+        for (; k + 16 <= kk; k += 16) {
+            const int64_t d = k + 8 * half;
+            float fa[FM][8], fb[FN][8];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                load_eight<AK>(fa[i], pa[i] + d * p.a_cs, p.a_cs);
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                load_eight<BK>(fb[j], pb[j] + d * p.b_rs, p.b_rs);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) {
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e],
+                                                                         acc[i][j], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll 1
+    for (; k < kk; k += 2) {
         const int64_t d = k + half;
         const bool inside = d < kk;
         float fa[FM], fb[FN];
@@ -486,12 +544,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
             squares_of[wave] = squares;
         }
         lds_barrier();
-        float most = 1.0f;
+        float all_squares = 0.0f;
 #pragma unroll
         for (int i = 0; i < kWaves; ++i) {
-            most += squares_of[i];
+            all_squares += squares_of[i];
         }
-        const float bound = 2.0f * most * static_cast<float>(kk) * 0x1p-97f;
+        const float bound = sums_bound(all_squares, kk);
         const Sums stand = judge(acc, bound);
         int under = 0;
         if (stand == Sums::kUnclear) {
@@ -525,8 +583,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void sgemm_split_kernel(Gem
             }
         }
         if (__builtin_amdgcn_readfirstlane(stand == Sums::kNotFinite || under > 0) != 0) {
-            plain_blocks<FM, FN>(acc, a_base, b_base, p, kk, w.rows_a, w.rows_b, wave_m * WM,
-                                 wave_n * WN, half, r32);
+            plain_blocks<FM, FN, AK, BK>(acc, a_base, b_base, p, kk, w.rows_a, w.rows_b,
+                                         wave_m * WM, wave_n * WN, half, r32);
         }
     }
     finish_tile<BM, BN, WM, WN, FM, FN>(acc, p, w, wave_m, wave_n, half, r32, gelu_table);
@@ -750,7 +808,7 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
     const int row0 = 32 * (set / FN);
     const int col0 = 32 * (set % FN);
     floatx16 mine[1][1];
-    float most = 1.0f;
+    float all_squares = 0.0f;
     if (has) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -764,9 +822,9 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
     }
 #pragma unroll
     for (int i = 0; i < WAVES_K; ++i) {
-        most += squares_of[i];
+        all_squares += squares_of[i];
     }
-    const float bound = 2.0f * most * static_cast<float>(kk) * 0x1p-97f;
+    const float bound = sums_bound(all_squares, kk);
     Sums stand = Sums::kClear;
     int under = 0;
     if (has && steps > 0) {
@@ -785,15 +843,16 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
         StepLoader<FM, AK> ra(a_base, p.a_rs, p.a_cs, w.rows_a, set, half, r32);
         StepLoader<FN, BK> rb(b_base, p.b_cs, p.b_rs, w.rows_b, set, half, r32);
         uint32_t found = 0xffffffffu;
-        for (int64_t t = set; t < steps; t += WAVES_K) {
-            const int64_t k_left = kk - 16 * t;
-            if (k_left >= 16) {
-                ra.template load<true>(0, k_left, WAVES_K, half);
-                rb.template load<true>(0, k_left, WAVES_K, half);
-            } else {
-                ra.template load<false>(0, k_left, WAVES_K, half);
-                rb.template load<false>(0, k_left, WAVES_K, half);
-            }
+        int64_t k_left = kk - 16 * set;
+#pragma unroll 4
+        for (; k_left >= 16; k_left -= 16 * WAVES_K) { // several steps' loads in flight
+            ra.template load<true>(0, k_left, WAVES_K, half);
+            rb.template load<true>(0, k_left, WAVES_K, half);
+            found = min(found, min(ra.smallest(), rb.smallest()));
+        }
+        if (k_left > 0) {
+            ra.template load<false>(0, k_left, WAVES_K, half);
+            rb.template load<false>(0, k_left, WAVES_K, half);
             found = min(found, min(ra.smallest(), rb.smallest()));
         }
         atomicMin(&smallest, found);
@@ -806,7 +865,7 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
         return;
     }
     if (__builtin_amdgcn_readfirstlane(stand == Sums::kNotFinite || under > 0) != 0) {
-        plain_blocks<1, 1>(mine, a_base, b_base, p, kk, w.rows_a, w.rows_b, row0, col0, half, r32);
+        plain_blocks<1, 1, AK, BK>(mine, a_base, b_base, p, kk, w.rows_a, w.rows_b, row0, col0, half, r32);
     }
     finish_tile<BM, BN, 32, 32, 1, 1>(mine, p, w, set / FN, set % FN, half, r32, gelu_table);
 }

@@ -53,7 +53,8 @@ def test_normal_operands(stream, tile, m, n, k):
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("case", ["inf", "inf times zero", "nan", "huge", "overflow", "tiny",
                                   "tiny and large", "tiny product", "denormal", "zero rows",
-                                  "zeros", "few tiny", "identity"])
+                                  "zeros", "few tiny", "identity", "zero rows, tiny columns",
+                                  "tiny by ordinary", "one tiny row"])
 def test_extreme_operands(stream, tile, case):
     # 16 x 16 tiles of 64x64: the register form; fewer workgroups than half the CUs: the other.
     for m, n, k in ((1000, 1000, 71), (150, 90, 200)):
@@ -85,6 +86,12 @@ def test_extreme_operands(stream, tile, case):
             a[:] = 0.0
         elif case == "few tiny":  # sums clear of what the tiny elements can lose
             a[:, 1::3] = normal((m, k), 5, 1e-39)[:, 1::3]
+        elif case == "zero rows, tiny columns":
+            a[m // 3: m // 2], b[:, ::5] = 0.0, b[:, ::5] * np.float32(1e-38)
+        elif case == "tiny by ordinary":
+            a = normal((m, k), 3, 1e-20)
+        elif case == "one tiny row":
+            a[7] *= np.float32(1e-37)
         elif case == "identity":  # every element comes back exactly
             b = np.zeros((k, n), np.float32)
             b[np.arange(min(k, n)), np.arange(min(k, n))] = 1.0
