@@ -443,7 +443,7 @@ void run_attention(mfr_stream& s, const mfr_attention_desc& d) {
     const int64_t block_q = 32 * waves; // queries per workgroup
     const int64_t q_blocks = (d.lq + block_q - 1) / block_q;
     const int64_t blocks = q_blocks * batch_count;
-    require(blocks < (int64_t{1} << 31), "attention: problem too large for one launch");
+    require(mfr::one_launch(blocks, 64 * waves), "attention: problem too large for one launch");
     p.q_blocks = static_cast<int32_t>(q_blocks);
     const unsigned grid = static_cast<unsigned>(blocks);
     if (d.d % 32 == 0) {

@@ -270,7 +270,8 @@ void run_decode(mfr_stream& s, const AttnParams& p, int64_t d) {
         }
     }
     const int64_t blocks = p.batch_count * ranges;
-    mfr::require(blocks < (int64_t{1} << 31) && p.batch_count * p.lq < (int64_t{1} << 31),
+    mfr::require(mfr::one_launch(blocks, kWaves * 64) &&
+                     (ranges == 1 || mfr::one_launch(p.batch_count * p.lq, 128)),
                  "attention: problem too large for one launch");
     const unsigned grid = static_cast<unsigned>(blocks);
     const int depth = static_cast<int>(d);

@@ -122,6 +122,15 @@ inline mfr_stream& stream_of(mfr_stream_t s) {
     return *s;
 }
 
+// Whether `blocks` workgroups of `threads` go in one launch: a launch of 2^32 threads or more runs
+// only what is left of it modulo 2^32 and reports nothing.
+constexpr bool one_launch(int64_t blocks, int64_t threads) {
+    return blocks < (int64_t{1} << 32) / threads;
+}
+
+// Rows that kernels of at most 64 threads a row take per launch.
+constexpr int64_t kLaunchRows = int64_t{1} << 25;
+
 inline unsigned grid_blocks(int64_t work, int64_t per_block, int64_t cap = int64_t{1} << 30) {
     int64_t blocks = (work + per_block - 1) / per_block;
     if (blocks < 1) {

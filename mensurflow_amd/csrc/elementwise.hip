@@ -9,6 +9,7 @@
 
 #include <type_traits>
 
+#include <algorithm>
 #include <cmath>
 
 namespace {
@@ -600,38 +601,38 @@ __global__ __launch_bounds__(256) void softmax_lines_kernel(const float* __restr
                                                             float* __restrict__ y, int64_t outer,
                                                             int64_t length, int64_t inner) {
     const int lane = threadIdx.x % kWave;
-    const int64_t line = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) +
-                         threadIdx.x / kWave;
-    if (line >= outer * inner) {
-        return;
-    }
-    const int64_t base = (line / inner) * length * inner + line % inner;
-    const float* in = x + base;
-    float* out = y + base;
-    float m = -INFINITY;
-    int has_nan = 0;
-    for (int64_t j = lane; j < length; j += kWave) {
-        const float v = in[j * inner];
-        has_nan |= __builtin_isnan(v) ? 1 : 0;
-        m = fmaxf(m, v);
-    }
-    m = line_max(mfr::dev::wave_max(m), mfr::dev::wave_or(has_nan));
-    if (m == -INFINITY) {
+    const int64_t waves = static_cast<int64_t>(gridDim.x) * (blockDim.x / kWave);
+    for (int64_t line = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) +
+                        threadIdx.x / kWave;
+         line < outer * inner; line += waves) {
+        const int64_t base = (line / inner) * length * inner + line % inner;
+        const float* in = x + base;
+        float* out = y + base;
+        float m = -INFINITY;
+        int has_nan = 0;
         for (int64_t j = lane; j < length; j += kWave) {
-            out[j * inner] = 0.0f;
+            const float v = in[j * inner];
+            has_nan |= __builtin_isnan(v) ? 1 : 0;
+            m = fmaxf(m, v);
         }
-        return;
-    }
-    double sum = 0.0;
-    for (int64_t j = lane; j < length; j += kWave) {
-        const float e = expf(in[j * inner] - m);
-        out[j * inner] = e;
-        sum += static_cast<double>(e);
-    }
-    sum = mfr::dev::wave_sum(sum);
-    const float scale = static_cast<float>(1.0 / sum);
-    for (int64_t j = lane; j < length; j += kWave) {
-        out[j * inner] = out[j * inner] * scale;
+        m = line_max(mfr::dev::wave_max(m), mfr::dev::wave_or(has_nan));
+        if (m == -INFINITY) {
+            for (int64_t j = lane; j < length; j += kWave) {
+                out[j * inner] = 0.0f;
+            }
+            continue;
+        }
+        double sum = 0.0;
+        for (int64_t j = lane; j < length; j += kWave) {
+            const float e = expf(in[j * inner] - m);
+            out[j * inner] = e;
+            sum += static_cast<double>(e);
+        }
+        sum = mfr::dev::wave_sum(sum);
+        const float scale = static_cast<float>(1.0 / sum);
+        for (int64_t j = lane; j < length; j += kWave) {
+            out[j * inner] = out[j * inner] * scale;
+        }
     }
 }
 
@@ -976,7 +977,7 @@ int mfr_where_nd(mfr_stream_t stream, int32_t ndim, const int64_t* shape, const 
         // R rows per workgroup along x; a row's columns in 256-thread chunks along y.
         const auto grid = [&](int rows_per_group) {
             const int64_t row_groups = (l.rows + rows_per_group - 1) / rows_per_group;
-            mfr::require(row_groups < (int64_t{1} << 31), "where_nd: too many rows");
+            mfr::require(mfr::one_launch(row_groups, 256), "where_nd: too many rows");
             const int64_t columns = quads ? l.row_len / 4 : l.row_len;
             const int64_t chunks = (columns + 255) / 256;
             return dim3(static_cast<unsigned>(row_groups),
@@ -1028,8 +1029,41 @@ int mfr_where_nd(mfr_stream_t stream, int32_t ndim, const int64_t* shape, const 
     });
 }
 
-// A workgroup of up to 1024 threads per row, fewer than 2^32 threads in a launch.
+// Rows that a workgroup of up to 1024 threads each takes in one launch.
 constexpr int64_t kBlockRows = int64_t{1} << 22;
+
+// Lines of `length` values `inner` apart; at most kLaunchRows of them where inner == 1.
+static void launch_softmax(mfr_stream& s, const float* x, float* y, int64_t outer, int64_t length,
+                           int64_t inner) {
+    const int64_t lines = outer * inner;
+    const unsigned blocks = mfr::grid_blocks(lines, 4, mfr::kLaunchRows / 4);
+    // Outputs past the last-level cache stream (512 MiB: 182 -> 178 us).
+    const bool stream_out =
+        4.0 * static_cast<double>(lines) * length > mfr::kLastLevelCacheBytes;
+    if (inner == 1 && length <= 64 * 4) {
+        softmax_rows_reg_kernel<4, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+    } else if (inner == 1 && length <= 64 * 16 && stream_out) {
+        softmax_rows_reg_kernel<16, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+    } else if (inner == 1 && length <= 64 * 16) {
+        softmax_rows_reg_kernel<16, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+    } else if (inner == 1 && length <= 64 * 32 && stream_out) {
+        softmax_rows_reg_kernel<32, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+    } else if (inner == 1 && length <= 64 * 32) {
+        softmax_rows_reg_kernel<32, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
+    } else if (inner == 1 && length <= 4 * 256 * 8 && lines < kBlockRows) {
+        softmax_block_kernel<256, 8><<<static_cast<unsigned>(lines), 256, 0, s.stream>>>(
+            x, y, length);
+    } else if (inner == 1 && length <= 4 * 1024 * 4 && lines < kBlockRows) {
+        softmax_block_kernel<1024, 4><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
+            x, y, length);
+    } else if (inner == 1 && length <= 4 * 1024 * 8 && lines < kBlockRows) {
+        softmax_block_kernel<1024, 8><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
+            x, y, length);
+    } else {
+        softmax_lines_kernel<<<blocks, 256, 0, s.stream>>>(x, y, outer, length, inner);
+    }
+    mfr::check_launch("softmax_kernel");
+}
 
 int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, int64_t length,
                 int64_t inner) {
@@ -1041,33 +1075,14 @@ int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, in
             return;
         }
         mfr::require(x != nullptr && y != nullptr, "softmax: null pointer");
-        const unsigned blocks = mfr::grid_blocks(lines, 4);
-        // Outputs past the last-level cache stream (512 MiB: 182 -> 178 us).
-        const bool stream_out =
-            4.0 * static_cast<double>(lines) * length > mfr::kLastLevelCacheBytes;
-        if (inner == 1 && length <= 64 * 4) {
-            softmax_rows_reg_kernel<4, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 64 * 16 && stream_out) {
-            softmax_rows_reg_kernel<16, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 64 * 16) {
-            softmax_rows_reg_kernel<16, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 64 * 32 && stream_out) {
-            softmax_rows_reg_kernel<32, true><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 64 * 32) {
-            softmax_rows_reg_kernel<32, false><<<blocks, 256, 0, s.stream>>>(x, y, lines, length);
-        } else if (inner == 1 && length <= 4 * 256 * 8 && lines < kBlockRows) {
-            softmax_block_kernel<256, 8><<<static_cast<unsigned>(lines), 256, 0, s.stream>>>(
-                x, y, length);
-        } else if (inner == 1 && length <= 4 * 1024 * 4 && lines < kBlockRows) {
-            softmax_block_kernel<1024, 4><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
-                x, y, length);
-        } else if (inner == 1 && length <= 4 * 1024 * 8 && lines < kBlockRows) {
-            softmax_block_kernel<1024, 8><<<static_cast<unsigned>(lines), 1024, 0, s.stream>>>(
-                x, y, length);
-        } else {
-            softmax_lines_kernel<<<blocks, 256, 0, s.stream>>>(x, y, outer, length, inner);
+        if (inner != 1) {
+            launch_softmax(s, x, y, outer, length, inner);
+            return;
         }
-        mfr::check_launch("softmax_kernel");
+        for (int64_t l = 0; l < lines; l += mfr::kLaunchRows) {
+            launch_softmax(s, x + l * length, y + l * length, std::min(lines - l, mfr::kLaunchRows),
+                           length, 1);
+        }
     });
 }
 
@@ -1077,6 +1092,23 @@ int mfr_softmax(mfr_stream_t stream, const float* x, float* y, int64_t outer, in
 // against 161; but 16384 x 4096: 62 -> 38, 32768 x 3500: 10 % faster).
 constexpr int64_t argmax_wide(int64_t rows) { return rows <= 4096 ? 1024 : 3072; }
 
+// At most kLaunchRows rows.
+static void launch_argmax(mfr_stream& s, const float* x, int64_t* out, int64_t rows,
+                          int64_t width) {
+    if (width > argmax_wide(rows) && width < (int64_t{1} << 31) - 65536 &&
+        rows < kBlockRows) {
+        const unsigned grid = static_cast<unsigned>(rows);
+        if (width <= 8192) {
+            argmax_block_kernel<256><<<grid, 256, 0, s.stream>>>(x, out, width);
+        } else {
+            argmax_block_kernel<1024><<<grid, 1024, 0, s.stream>>>(x, out, width);
+        }
+    } else {
+        argmax_kernel<<<mfr::grid_blocks(rows, 4), 256, 0, s.stream>>>(x, out, rows, width);
+    }
+    mfr::check_launch("argmax_kernel");
+}
+
 int mfr_argmax(mfr_stream_t stream, const float* x, int64_t* out, int64_t rows, int64_t width) {
     return mfr::guarded([&] {
         auto& s = mfr::stream_of(stream);
@@ -1085,18 +1117,10 @@ int mfr_argmax(mfr_stream_t stream, const float* x, int64_t* out, int64_t rows, 
             return;
         }
         mfr::require(out != nullptr && (width == 0 || x != nullptr), "argmax: null pointer");
-        if (width > argmax_wide(rows) && width < (int64_t{1} << 31) - 65536 &&
-            rows < kBlockRows) {
-            const unsigned grid = static_cast<unsigned>(rows);
-            if (width <= 8192) {
-                argmax_block_kernel<256><<<grid, 256, 0, s.stream>>>(x, out, width);
-            } else {
-                argmax_block_kernel<1024><<<grid, 1024, 0, s.stream>>>(x, out, width);
-            }
-        } else {
-            argmax_kernel<<<mfr::grid_blocks(rows, 4), 256, 0, s.stream>>>(x, out, rows, width);
+        for (int64_t r = 0; r < rows; r += mfr::kLaunchRows) {
+            launch_argmax(s, x != nullptr ? x + r * width : nullptr, out + r,
+                          std::min(rows - r, mfr::kLaunchRows), width);
         }
-        mfr::check_launch("argmax_kernel");
     });
 }
 

@@ -404,8 +404,7 @@ void launch_split(int tile, const GemmParams& q, bool ak, bool bk, unsigned bloc
     case MFR_TILE_128x64: launch_split_128x64(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x128: launch_split_64x128(q, ak, bk, blocks, stream); break;
     case MFR_TILE_64x64:
-        // (512 threads a workgroup, fewer than 2^32 in a launch.)
-        if (q.m <= kFewRows && near && blocks < (1u << 23) &&
+        if (q.m <= kFewRows && near && mfr::one_launch(blocks, 512) &&
             few_rows_form(blocks, q.k_per_split, q.splits, bk, cus)) {
             launch_split_regs_32x64(q, ak, bk, blocks, stream);
         } else if (q.splits == 1 && regs_form(blocks, q.k, cus) && near) {
@@ -447,11 +446,12 @@ struct StageBatch {
 
 // dst line r (r = matrix * lines + line, matrices in the order of StageBatch) gets the `inner`
 // unit-stride floats of source line `line` of that matrix, then zeros up to `pitch` (a multiple
-// of 4); dst is 16-byte aligned and matrix-contiguous. One workgroup per line.
+// of 4); dst is 16-byte aligned and matrix-contiguous. One workgroup per line, from line `first` on.
 __global__ __launch_bounds__(256) void stage_kernel(const float* src, float* dst, int64_t lines,
                                                     int64_t inner, int64_t line_stride,
-                                                    int64_t pitch, StageBatch sb) {
-    const int64_t r = blockIdx.x;
+                                                    int64_t pitch, StageBatch sb,
+                                                    int64_t first) {
+    const int64_t r = first + blockIdx.x;
     int64_t matrix = r / lines;
     const int64_t line = r - matrix * lines;
     int64_t offset = line * line_stride;
@@ -513,10 +513,12 @@ void stage_operand(Operand& o, float* dst, const GemmParams& p, hipStream_t stre
         }
     }
     const int64_t rows = matrices * o.lines;
-    mfr::require(rows < (int64_t{1} << 31), "sgemm: operand too large to stage");
-    stage_kernel<<<static_cast<unsigned>(rows), 256, 0, stream>>>(o.base, dst, o.lines, o.inner,
-                                                                  *o.line_stride, pitch, sb);
-    mfr::check_launch("stage_kernel");
+    constexpr int64_t kPerLaunch = int64_t{1} << 23; // one_launch
+    for (int64_t r = 0; r < rows; r += kPerLaunch) {
+        stage_kernel<<<static_cast<unsigned>(std::min(rows - r, kPerLaunch)), 256, 0, stream>>>(
+            o.base, dst, o.lines, o.inner, *o.line_stride, pitch, sb, r);
+        mfr::check_launch("stage_kernel");
+    }
     repoint_staged(o, dst, p);
 }
 
@@ -950,7 +952,9 @@ void launch_thin(const Plan& plan, const GemmParams& q, int va, int vb, hipStrea
     mfr::require(stage == nullptr || (along_n && width == 1 && q.batch_count == 1),
                  "sgemm: the strip stages A only from 4-byte rows of one matrix");
     const int64_t blocks = t.blocks_per_batch * q.batch_count;
-    mfr::require(blocks < (int64_t{1} << 31), "sgemm: problem too large for one launch");
+    mfr::require(mfr::one_launch(blocks, kThinThreads) &&
+                     (stage == nullptr || mfr::one_launch(t.rows, 64)),
+                 "sgemm: problem too large for one launch");
     const unsigned grid = static_cast<unsigned>(blocks);
     // The column count rounded up to 1, 2, 4 or 8 (kThinCols).
     const int c = t.cols <= 1 ? 1 : t.cols <= 2 ? 2 : t.cols <= 4 ? 4 : kThinCols;
@@ -1073,7 +1077,8 @@ void launch_region(const Plan& plan, const GemmParams& p, const Region& r, int v
     const int64_t tiles_n = (q.n + kTiles[tile].bn - 1) / kTiles[tile].bn;
     const int64_t blocks = tiles_m * tiles_n * q.batch_count * r.splits;
     require(tiles_m < (int64_t{1} << 30) && tiles_n < (int64_t{1} << 30) &&
-                blocks < (int64_t{1} << 31),
+                mfr::one_launch(blocks, tile == MFR_TILE_256x256 || tile == MFR_TILE_128x128 ? 512
+                                                                                             : 256),
             "sgemm: problem too large for one launch");
     q.tiles_m = static_cast<int32_t>(tiles_m);
     q.tiles_n = static_cast<int32_t>(tiles_n);

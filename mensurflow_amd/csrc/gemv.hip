@@ -31,6 +31,8 @@
 // 67.5 -> 17.3, 16383 x 16381 908 -> 172 (one float per lane before).
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace {
 
 using mfr::dev::kWave;
@@ -396,12 +398,12 @@ int64_t t_rows_per_chunk(int64_t rows, int64_t strips) {
 }
 
 // The N form's kernel: the streaming kernel (8 rows per wavefront, aligned rows) where it gives
-// every CU 4 wavefronts; else from 2048 rows on 4 rows per workgroup (or the narrow kernel where
+// every CU 4 wavefronts, or where there are too few columns for four to share (8188 x 512: 4.65 us,
+// the narrow kernel 4.94); else from 2048 rows on 4 rows per workgroup (or the narrow kernel where
 // the columns do not feed four wavefronts), below that one.
 constexpr int64_t kStreamRows = 8192;
 constexpr int64_t kSharedRows = 2048;
 constexpr int64_t kNarrowCols = 512;
-constexpr int64_t kManyRows = int64_t{1} << 24; // past this only 16 threads a row fit a launch
 
 void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float alpha,
                  const float* a, int64_t lda, const float* x, float beta, const float* y0,
@@ -419,12 +421,20 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
     mfr::require(inputs == 0 || (a != nullptr && x != nullptr), "gemv: null A or x");
     const bool vec4 = mfr::aligned16(a) && lda % 4 == 0 && cols % 4 == 0 &&
                       (!trans ? mfr::aligned16(x) : true);
+    if (!trans && rows > mfr::kLaunchRows) {
+        for (int64_t r = 0; r < rows; r += mfr::kLaunchRows) {
+            launch_gemv(s, false, std::min(rows - r, mfr::kLaunchRows), cols, alpha,
+                        a != nullptr ? a + r * lda : nullptr, lda, x, beta,
+                        y0 != nullptr ? y0 + r : nullptr, y + r);
+        }
+        return;
+    }
     if (!trans) {
         if (vec4 && (rows >= kStreamRows || (rows >= kSharedRows && cols <= kNarrowCols))) {
             const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
             gemv_n_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN), kWave * kWavesPerBlockN, 0,
                             s.stream>>>(a, lda, x, rows, cols, alpha, beta, y0, y);
-        } else if (rows >= kSharedRows && (cols <= kNarrowCols || rows >= kManyRows)) {
+        } else if (rows >= kSharedRows && cols <= kNarrowCols) {
             const int64_t waves = (rows + kRowsPerWave - 1) / kRowsPerWave;
             gemv_n_narrow_kernel<<<mfr::grid_blocks(waves, kWavesPerBlockN),
                                    kWave * kWavesPerBlockN, 0, s.stream>>>(
@@ -442,7 +452,7 @@ void launch_gemv(mfr_stream& s, bool trans, int64_t rows, int64_t cols, float al
     const int64_t strips = (cols + kStripCols - 1) / kStripCols;
     const int64_t per = rows > 0 ? t_rows_per_chunk(rows, strips) : 1;
     const int64_t chunks = rows > 0 ? (rows + per - 1) / per : 0;
-    mfr::require(strips < (int64_t{1} << 31) && chunks < 65536, "gemv: matrix too large");
+    mfr::require(mfr::one_launch(strips, kWave) && chunks < 65536, "gemv: matrix too large");
     double* partial = nullptr;
     // Held until both kernels are queued: another thread's reserve() may not free `partial`
     // in between.
@@ -546,7 +556,7 @@ void launch_dot(mfr_stream& s, int64_t n, const float* x, const float* y, float*
     mfr::require(out != nullptr, "dot: null out");
     mfr::require(n == 0 || (x != nullptr && y != nullptr), "dot: null x or y");
     const int64_t chunks = (n + kDotChunk - 1) / kDotChunk;
-    mfr::require(chunks < (int64_t{1} << 31), "dot: vector too long");
+    mfr::require(mfr::one_launch(chunks, kDotThreads), "dot: vector too long");
     // Held until both kernels are queued (another thread's reserve() may not free `partial`).
     std::lock_guard<std::mutex> hold(s.workspace_mutex);
     double* partial = nullptr;

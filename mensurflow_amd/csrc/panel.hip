@@ -38,7 +38,7 @@ void launch_panel(const GemmParams& q, bool nt, int cus, hipStream_t stream) {
     const int64_t per_chunk = (nblocks + chunks - 1) / chunks;
     chunks = (nblocks + per_chunk - 1) / per_chunk;
     const int64_t blocks = owners * chunks;
-    mfr::require(blocks < (int64_t{1} << 31) && nblocks < (int64_t{1} << 30),
+    mfr::require(mfr::one_launch(blocks, kPanelThreads) && nblocks < (int64_t{1} << 30),
                  "sgemm: problem too large for one launch");
     pp.panels = static_cast<int32_t>(panels);
     pp.nblocks = static_cast<int32_t>(nblocks);

@@ -112,3 +112,61 @@ def test_streamed_output_past_last_level_cache(stream):
         assert same_bits(wide.slice(0, lo, lo + 3).numpy()[:, :n], want), lo
     c.close()
     wide.close()
+
+
+def test_rows_past_one_launch(stream):
+    """A launch holds fewer than 2^32 threads: gemv N over 2^29 + 9 rows (8 threads each), argmax and
+    softmax over 2^26 + 5 lines (64 threads each) reach their last rows, softmax along either axis."""
+    rows = (1 << 29) + 9
+    a = mf.DeviceArray.empty((rows, 1), stream)
+    y = mf.DeviceArray.empty((rows,), stream)
+    mf.fill(a, 2.0)
+    mf.fill(y, 7.0)
+    mf.sgemv(a, dev(np.array([3.0], np.float32), stream), out=y)
+    for lo in (0, rows // 2, rows - 1000):
+        assert np.all(y.slice(0, lo, lo + 1000).numpy() == 6.0), lo
+    a.close()
+    y.close()
+    lines = (1 << 26) + 5
+    x = mf.DeviceArray.empty((lines, 2), stream)
+    mf.fill(x, 1.0)
+    mf.fill(x.slice(0, lines - 1, lines).slice(1, 1, 2).view((1,)), 2.0)
+    index = mf.DeviceArray.empty((lines,), stream, np.int64)
+    mf.fill(index, 9)
+    mf.argmax(x, out=index)
+    tail = index.slice(0, lines - 1000, lines).numpy()
+    assert np.all(tail[:-1] == 0) and tail[-1] == 1
+    p = mf.DeviceArray.empty((lines, 2), stream)
+    mf.fill(p, 7.0)
+    mf.softmax(x, out=p)
+    assert np.all(p.slice(0, lines - 1000, lines - 1).numpy() == 0.5)
+    mf.fill(x, 1.0)
+    mf.fill(p, 7.0)
+    columns = x.view((2, lines))
+    mf.softmax(columns, axis=0, out=p.view((2, lines)))
+    assert np.all(p.slice(0, lines - 1000, lines).numpy() == 0.5)
+
+
+def test_too_many_workgroups_are_refused(stream):
+    """Products and heads that would need 2^32 threads in one launch are errors, and write nothing."""
+    c = mf.DeviceArray.empty((1024,), stream)
+    mf.fill(c, 7.0)
+    x = dev(np.ones(4096, np.float32), stream)
+    d = mf.GemmDesc()
+    d.m = d.n = d.k = d.a_rs = d.a_cs = d.b_rs = d.b_cs = d.c_rs = 1
+    d.batch_dims, d.alpha, d.tile = 2, 1.0, mf.abi.TILE_64x64
+    d.batch[0], d.batch[1] = 1 << 12, 1 << 12
+    d.a = d.b = x.ptr
+    d.c = c.ptr
+    with pytest.raises(ValueError):
+        mf.sgemm(stream, d)
+    q = mf.abi.AttentionDesc()
+    q.lq, q.lk, q.d, q.batch_dims = 8, 8, 64, 2
+    q.batch[0], q.batch[1] = 1 << 12, 1 << 12
+    for name in ("q", "k", "v", "out"):
+        setattr(q, name, x.ptr)
+        setattr(q, name + "_rs", 64)
+    with pytest.raises(ValueError):
+        import ctypes
+        mf.abi.check(mf.abi.load().mfr_attention(stream.handle, ctypes.byref(q)), "mfr_attention")
+    assert np.all(c.numpy() == 7.0) and np.all(x.numpy() == 1.0)
