@@ -622,7 +622,7 @@ void consider_peeling(Plan& plan, int64_t batch, int cus, double single_us) {
         const int64_t rem_m = p.m % bm, rem_n = p.n % bn;
         const bool peel_m = p.m > bm && rem_m > 0 && rem_m * 4 <= bm;
         const bool peel_n = p.n > bn && rem_n > 0 && rem_n * 4 <= bn;
-        if (!peel_m && !peel_n) {
+        if ((!peel_m && !peel_n) || (t == MFR_TILE_256x256 && !big_tile_ok(plan))) {
             continue;
         }
         const int64_t main_m = peel_m ? p.m - rem_m : p.m;
@@ -701,6 +701,9 @@ bool panel_fits(const Plan& plan) {
         return false;
     }
     if (p.k < 1 || p.k > kPanelMaxDepth || p.act != MFR_ACT_NONE) {
+        return false;
+    }
+    if (p.a_rs < 0 || p.b_cs < 0) { // its buffer resources start at the first row
         return false;
     }
     const double limit = 2147483648.0;

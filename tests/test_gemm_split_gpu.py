@@ -132,11 +132,13 @@ def test_no_larger_error_than_fp32_chains(stream):
             assert rel <= np.sqrt(k) * 2.0**-24 * 0.3, (k, tile, rel)
 
 
-@pytest.mark.parametrize("m,n,k", [(256, 256, 256), (20, 250, 500), (200, 250, 71), (130, 70, 40)])
+@pytest.mark.parametrize("m,n,k", [(256, 256, 256), (20, 250, 500), (200, 250, 71), (130, 70, 40),
+                                   (300, 260, 71), (2100, 2100, 40)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 def test_lines_that_run_backwards(stream, m, n, k, ta, tb):
     """Operands whose lines lie a negative stride apart (the descriptor takes any element strides):
-    quarter integers, so the product is exact on AUTO and on every tile."""
+    quarter integers, so the product is exact on AUTO (which would peel a strip off a 256x256 tile, or take the panel path,
+    were the lines in order) and on every tile."""
     a, b = quarter_matrix(m, k, 1), quarter_matrix(k, n, 2)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
     # Stored along k or along m (n), the lines in reverse order.
