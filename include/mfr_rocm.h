@@ -124,8 +124,11 @@ int mfr_event_elapsed_ms(mfr_event_t start, mfr_event_t end, float* ms);
  * transposed); C has column stride 1. c0 may equal c (in place). k == 0 gives the epilogue of
  * a zero product. The products are summed in fp32 on the matrix cores, in a different order from
  * the CPU's packed kernel: up to a depth of 64 as fp32 products (v_mfma_f32_32x32x2_f32), above
- * it as the six products of three-way bf16 parts that reach fp32 precision (their error against
- * 64 bits is below the fp32 products'; what the parts cannot hold runs as fp32 products).
+ * it as the six products of three-way bf16 parts that reach fp32 precision (what the parts cannot
+ * hold runs as fp32 products). A sum's error is at most (2 + 6 s) 2^-24 of sum |a b| there, s the
+ * 16-deep steps of the depth that hold nonzero products: on dense operands less than the fp32
+ * products' (2-norm 4.9e-7 against 5.8e-7 at a depth of 1024), on rows with few nonzeros or of widely
+ * differing sizes up to 1.75 times it (32 nonzeros of 4096: 1.2e-7 against 6.9e-8).
  *
  * Replaces: the Matmul kernel (src/backends/cpu/backend.cpp:131-164), the GemmBatched kernel
  * (backend.cpp:239-291), and the 4-dispatch composition of mensurflow::gemm

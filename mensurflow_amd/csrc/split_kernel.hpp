@@ -1,11 +1,18 @@
 // The fp32 GEMM tile on the bf16 matrix cores: each fp32 operand element is cut exactly into three
 // bf16 parts (8 bits each) and the product is summed from the six part products that reach fp32
-// precision. The three left out are at most 2^-23 of |a b| together and 1.4e-8 of it root mean
-// square, under one fp32 rounding. Measured against 64 bits the sums are nearer than the fp32
-// matrix cores' (one rounding per 16 depths and part product, against one per depth): at a depth
-// of 64 / 1024 / 4096, uniform operands, 1.1e-7 / 4.6e-7 / 9.2e-7 against 1.5e-7 / 5.8e-7 /
-// 1.03e-6; normal 1.1e-7 / 4.9e-7 / 9.8e-7 against 1.4e-7 / 5.8e-7 / 1.1e-6; positive 8.4e-8 /
-// 2.8e-7 / 5.2e-7 against 1.1e-7 / 4.3e-7 / 8.9e-7.
+// precision (the method of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", ARITH 2019). The three left out are at
+// most 2^-24 of |a b| together and 1.4e-8 of it root mean square, and each 16 depths that hold
+// anything but zeros round the sum six times, where the fp32 matrix cores round it once per depth
+// and their products not at all. A sum of k products whose nonzero ones lie in s steps of 16 depths
+// is so within (2 + 6 s) 2^-24 of sum |a b| of the exact one, against k 2^-24.
+//
+// On dense operands that is nearer (2-norm error at a depth of 64 / 1024 / 4096: uniform 1.1e-7 /
+// 4.6e-7 / 9.2e-7 against 1.5e-7 / 5.8e-7 / 1.03e-6 on the fp32 matrix cores; normal 1.1e-7 / 4.9e-7 /
+// 9.8e-7 against 1.4e-7 / 5.8e-7 / 1.1e-6; positive 8.4e-8 / 2.8e-7 / 5.2e-7 against 1.1e-7 / 4.3e-7 /
+// 8.9e-7). On sparse or widely scaled rows it is further off: with 1 / 4 / 16 / 32 nonzeros in rows
+// of 512 / 512 / 1024 / 4096 3.5e-8 / 5.6e-8 / 9.1e-8 / 1.2e-7 against 2.5e-8 / 4.2e-8 / 5.9e-8 /
+// 6.9e-8, half zeros (1024 deep) 2.3e-7 against 2.1e-7, exp(2 N) times normal 2.4e-7 against 2.1e-7.
 // Included by the split_*.hip translation units (launches) through split.hpp; see gemm.hip for the
 // tiles, regions and splits around it.
 #pragma once

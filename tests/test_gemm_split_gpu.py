@@ -56,8 +56,9 @@ def test_normal_operands(stream, tile, m, n, k):
                                   "zeros", "few tiny", "identity", "zero rows, tiny columns",
                                   "tiny by ordinary", "one tiny row"])
 def test_extreme_operands(stream, tile, case):
-    # 16 x 16 tiles of 64x64: the register form; fewer workgroups than half the CUs: the other.
-    for m, n, k in ((1000, 1000, 71), (150, 90, 200)):
+    # 16 x 16 tiles of 64x64: the register form; fewer workgroups than half the CUs: the other; at
+    # most 32 rows: the 32x64 form, with and without its loop of two steps in flight.
+    for m, n, k in ((1000, 1000, 71), (150, 90, 200), (20, 150, 71), (20, 150, 500)):
         a, b = normal((m, k), 3), normal((k, n), 4)
         if case == "inf":
             a[5, 3], a[m - 1, k - 1], b[7, 11] = np.inf, -np.inf, np.inf
@@ -194,3 +195,59 @@ def test_few_rows_batched_exact(stream, batch, k):
         b_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(np.swapaxes(b, 1, 2) if tb else b), stream)
         mf.gemm_batched(a_d, b_d.transpose(-2, -1) if tb else b_d, c)
         assert np.array_equal(c.numpy(), want), tb
+
+
+@pytest.mark.parametrize("nonzeros,k", [(1, 512), (2, 512), (4, 512), (8, 1024), (32, 4096),
+                                        (500, 1000)])
+def test_sparse_and_wide_rows(stream, nonzeros, k):
+    """Rows with few nonzeros, and rows of widely differing sizes, within (2 + 6 s) 2^-24 of
+    sum |a b|: s steps of 16 depths with a nonzero, six roundings each, the products left out and the
+    last rounding."""
+    rng = np.random.default_rng(k)
+    sparse = np.zeros((200, k), np.float32)
+    for row in sparse:
+        row[rng.choice(k, nonzeros, replace=False)] = rng.standard_normal(nonzeros)
+    wide = (rng.standard_normal((200, k)) * np.exp(3 * rng.standard_normal((200, k)))).astype(np.float32)
+    b = normal((k, 150), 2)
+    for a in (sparse, wide):
+        padded = np.pad(a != 0, ((0, 0), (0, -k % 16))).reshape(200, -1, 16)
+        steps = padded.any(axis=2).sum(axis=1)[:, None]
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        scale = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+        for tile in TILES:
+            got = mf.gemm(mf.DeviceArray.from_numpy(a, stream),
+                          mf.DeviceArray.from_numpy(b, stream), tile=tile, splits=1).numpy()
+            assert np.all(np.abs(got - want) <= (2 + 6 * steps) * 2.0**-24 * scale), tile
+            if a is sparse:
+                # One rounding for a nonzero's own products and six a step that add up as their root:
+                # at most 2^-24 each, 0.58 of it root mean square where the adder truncates, times
+                # the share of a partial sum in the whole (0.71 on average). 0.40 is measured.
+                rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+                assert rel <= 0.5 * 2.0**-24 * np.sqrt(1 + 6 * min(nonzeros, k // 16 + 1)), tile
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 300, 1000), (20, 130, 400), (32, 513, 4096), (64, 64, 1024),
+                                   (200, 130, 500)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_every_part_counts(stream, m, n, k, ta, tb):
+    """AUTO and many depth ranges in every layout, full mantissas: the 2-norm error stays under 0.3
+    sqrt(k) 2^-24 (test_no_larger_error_than_fp32_chains), where losing the third part of either
+    operand (2^-19 of it root mean square) alone would be 1.9e-6, past the bound at any depth here."""
+    a, b = normal((m, k), 13), normal((k, n), 14)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    a_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(a.T if ta else a), stream)
+    b_d = mf.DeviceArray.from_numpy(np.ascontiguousarray(b.T if tb else b), stream)
+    for tile, splits in ((0, 0), (0, 1), (mf.abi.TILE_64x64, 12), (mf.abi.TILE_128x64, 3)):
+        got = mf.gemm(a_d, b_d, trans_a=ta, trans_b=tb, tile=tile, splits=splits).numpy()
+        rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert rel <= 0.3 * np.sqrt(k) * 2.0**-24, (tile, splits, rel)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_identity_gives_b_exactly(stream, tile):
+    """The identity times b: every part of b counts (test_extreme_operands has a times it)."""
+    for m, n in ((300, 260), (20, 150), (130, 70)):
+        b = normal((m, n), 15)
+        got = mf.gemm(mf.DeviceArray.from_numpy(np.eye(m, dtype=np.float32), stream),
+                      mf.DeviceArray.from_numpy(b, stream), tile=tile, splits=1).numpy()
+        assert np.array_equal(got, b)
