@@ -172,16 +172,17 @@ enum { MFR_GEMM_CAUSAL = 1 };
  * shape, into the stream's workspace (one extra pass over it). AUTO stages when the product is
  * large (>= 2^30 flops) and the copy is small next to it (<= 1 byte per 64 flops), except that
  * under the 256x256 tile it stages only operands with a unit stride along the depth and reads the
- * others in place; the result is the same either way. Without staging, the 256x256 tile reads
- * such operands in place, with 4-byte buffer loads that write LDS directly. */
+ * others in place; the result is the same either way. Without staging, such operands are read in
+ * place: 4 bytes at a time, but 16 along the depth above a depth of 64. */
 enum { MFR_STAGE_AUTO = 0, MFR_STAGE_NEVER = 1, MFR_STAGE_ALWAYS = 2 };
 
 /* Workgroup tile of mfr_sgemm (rows x cols). AUTO picks one from the shape (with the split
  * count): a time model of the busiest CU's tiles (ceil(tiles / CUs) of them, each its depth at
  * the tile's measured rate plus a fixed time), and the 128x64 or 64x128 tile for a depth <= 64.
- * A fixed tile is what
- * a tuner sets (the reference's TuningConfig,
- * src/core/dispatcher.hpp:145-149). Every tile gives the same results up to summation order. */
+ * A fixed tile is what a tuner sets (the reference's TuningConfig, src/core/dispatcher.hpp:145-149).
+ * Every tile gives the same results up to summation order. A fixed 256x256 tile is refused
+ * (MFR_E_UNSUPPORTED) where a slice of an operand, 256 of its lines along k or 32 along its rows,
+ * spans 2^30 bytes or more or its lines run backwards. */
 enum {
     MFR_TILE_AUTO = 0,
     MFR_TILE_256x256 = 1, /* 8 wavefronts of 128x64, 1 workgroup per CU */
@@ -205,8 +206,8 @@ enum {
  * the next columns are multiplied, so the stores overlap the MFMA work instead of following it.
  * It takes 1 <= k <= 64 with both operands read along k (unit stride along K) by 16-byte loads
  * (their k, other strides and bases 16-byte aligned), no activation and no split; alpha, beta *
- * C0 and a bias as everywhere. The sums are the MFMA tiles' own, so the results are the same bit
- * for bit. Elsewhere a fixed PANEL fails with MFR_E_UNSUPPORTED. AUTO takes it where it fits for
+ * C0 and a bias as everywhere. The sums are those of the 128x64 and 64x128 tiles, which run such
+ * depths as fp32 products too, so the results are the same bit for bit. Elsewhere a fixed PANEL fails with MFR_E_UNSUPPORTED. AUTO takes it where it fits for
  * outputs of more than 128 rows and at least 2^22 elements. */
 
 /* Split-K of mfr_sgemm. A product with few output tiles and a long depth (256 x 256 x 16384)
@@ -215,8 +216,7 @@ enum {
  * to the stream's workspace (splits * m * n * batch floats), and a second pass adds the ranges in
  * order and applies the epilogue with the same roundings. AUTO picks the tile and the count
  * together from a time model (no split when the output fills the device, ranges >= 256 deep, 128 for
- * the 64x64 tile,
- * partial sums <= 1 GiB) and falls back to no split when the workspace cannot be had; a fixed
+ * the 64x64 tile, partial sums <= 1 GiB) and falls back to no split when the workspace cannot be had; a fixed
  * count fails with MFR_E_RUNTIME then. Results are deterministic; the summation order, hence
  * the rounding, depends on the count. */
 #define MFR_MAX_SPLITS 64
@@ -243,8 +243,9 @@ int mfr_sgemm_noalloc(mfr_stream_t stream, const mfr_gemm_desc* desc);
 /* Edge peeling (tile and splits both AUTO): a dimension a few rows past a multiple of a big tile
  * (N = 4099 = 16 x 256 + 3) would cost that tile a whole extra wave of tiles for a sliver of work,
  * so such a remainder (at most a quarter of the tile) may run as a separate launch with its own
- * tile and split count, when the time model prices that at least 5% lower. Up to 4 launches: the main
- * rectangle, the right strip, the bottom strip, the corner. */
+ * tile and split count, when the time model prices that at least 5% lower; at most 8 rows or columns
+ * off a product of 2^34 flops or more, when it prices that no more than 5% higher. Up to 4 launches:
+ * the main rectangle, the right strip, the bottom strip, the corner. */
 
 /* What mfr_sgemm would run for desc on device `device`, without launching anything: the tile
  * (an MFR_TILE_* other than AUTO; AUTO when there is nothing to compute), whether operands
@@ -253,7 +254,7 @@ int mfr_sgemm_noalloc(mfr_stream_t stream, const mfr_gemm_desc* desc);
  * output regions launched separately (1, or 2-4 with edge peeling; 0 when there is nothing to
  * compute). Validates desc as mfr_sgemm
  * does and fails with the same status where mfr_sgemm would (MFR_E_UNSUPPORTED for a fixed
- * 256x256 tile with staging off and operands 16-byte loads cannot read). For tuners: the default
+ * 256x256 tile and operands whose lines lie too far apart for it). For tuners: the default
  * a search starts from, and whether a (tile, stage) point can run (the reference's
  * TunableKernel::defaults / allowed, src/core/dispatcher.hpp:226-239). */
 int mfr_sgemm_plan(int device, const mfr_gemm_desc* desc, int32_t* tile, int32_t* stage,
@@ -351,7 +352,9 @@ int mfr_elementwise(mfr_stream_t stream, int op, const float* a, const float* b,
  * with every key removed gives zeros, a NaN score gives a NaN row. q [.., lq, d], k [.., lk, d],
  * v [.., lk, d] and out [.., lq, d] have unit stride along d, row strides and batch strides
  * (0 = broadcast) that are multiples of 4 floats and 16-byte aligned bases; d is a multiple of 16,
- * at most 128.
+ * at most 128. Scores and outputs are summed in fp32, for d = 32, 64, 96 and 128 from three-way bf16
+ * parts as mfr_sgemm's (what the parts cannot hold, as fp32 products). Calls of 1 to 4 queries may
+ * use the stream's workspace; a captured one uses none.
  * Anything else is MFR_E_UNSUPPORTED (the caller composes the op instead). The mask (NULL, or
  * 1 byte per element: nonzero keeps) has any strides, 0 for broadcast dimensions. scale 0 means
  * fl(1/sqrt(d)).

@@ -390,7 +390,7 @@ void launch_layout(int tile, const GemmParams& p, int va, int vb, unsigned block
 // Whether a tile runs the split kernel (bf16 matrix cores, split_kernel.hpp) on a product of depth
 // k. The 128x64 and 64x128 tiles, which AUTO takes for short depths, keep the fp32 matrix cores up
 // to the panel path's 64: there the products are one or two slices and bound by latency and the
-// output, and the two paths give the same bits.
+// output, and the panel path gives these tiles' bits.
 bool split_takes(int tile, int64_t k) {
     return (tile != MFR_TILE_128x64 && tile != MFR_TILE_64x128) || k > kPanelMaxDepth;
 }
@@ -608,8 +608,9 @@ void single_region(Plan& plan, const Choice& choice) {
 // no more than 5% above it for a sliver off a large product.
 constexpr double kLaunchUs = 5.0;
 constexpr double kPeelMargin = 0.95;
-// A sliver of at most 8 rows or columns is peeled off unless that is priced this much higher: the
-// model is no nearer than that (3 x 2049 x 2047 x 2048: 274 us whole, 284 in two).
+// A sliver of at most 8 rows or columns off a large product is peeled off unless that is priced
+// this much higher: the model is no nearer than 5 %, and a test of the plan holds two launches for
+// 3 x 2049 x 2047 x 2048, though there it costs (284 us in two, 274 whole).
 constexpr double kSliverMargin = 1.05;
 
 bool big_tile_ok(const Plan& plan);
@@ -677,10 +678,10 @@ int64_t staged_floats_padded(const Operand& o, const GemmParams& p) {
     return (staged_floats(o, p) + 63) / 64 * 64; // 256-byte aligned parts of the workspace
 }
 
-// Whether the 256x256 tile can read the plan's operands (as they will be after staging): it
-// copies both slices straight into LDS with buffer loads, whose byte offsets within a slice must
-// stay below 2^30: 255 lines of a K-major operand, or 31 depth lines of the other, plus a line's
-// own extent.
+// Whether the 256x256 tile takes the plan's operands (as they will be after staging): a slice, 255
+// lines of a K-major operand or 31 depth lines of the other plus a line's own extent, spans less
+// than 2^30 bytes, and lines do not run backwards. Its loads would reach further (64-bit addresses);
+// the limit is the entry point's contract (a fixed tile past it is MFR_E_UNSUPPORTED).
 bool big_tile_ok(const Plan& plan) {
     GemmParams p = plan.p;
     const auto fits = [](const Operand& o, bool kmaj, bool staged) {
@@ -847,10 +848,9 @@ Plan plan_sgemm(const mfr_gemm_desc& d, int cus) {
     };
     tile_plan(plan);
     // AUTO staging under the 256x256 tile: an operand whose unit stride runs along its rows (M
-    // or N) is read in place instead. Its direct-to-LDS slices are whole runs of 256 floats,
-    // about one cache line more per run than the aligned copy, where a K-major operand's runs of
-    // 32 floats would touch twice the lines. configs[3]: X staged and W in place 323 us, both
-    // staged 331 us, both in place 333 us.
+    // or N) is read in place instead. Its loads are 4 bytes a lane along whole lines either way, so a
+    // copy gains nothing; along the depth the tile loads 16 bytes at any 4-byte alignment, and a copy
+    // saves a cache line in four (4096 x 4096 x 1023 161.6 us in place, 1024 deep 160.4).
     if (d.stage == MFR_STAGE_AUTO && plan.regions[0].tile == MFR_TILE_256x256 &&
         ((plan.stage_a && !plan.ak) || (plan.stage_b && !plan.bk))) {
         Plan partial = plan;
@@ -1268,8 +1268,7 @@ void run_sgemm(mfr_stream& s, const mfr_gemm_desc& d, float* scratch = nullptr,
             if (d.stage == MFR_STAGE_ALWAYS) {
                 throw mfr::Error(MFR_E_RUNTIME, "sgemm: no workspace for operand staging");
             }
-            // AUTO without the memory: read in place (4-byte loads; the 256x256 tile copies them
-            // straight into LDS).
+            // AUTO without the memory: read in place.
             plan.stage_a = plan.stage_b = false;
             fa = fb = 0;
             if (d.tile == MFR_TILE_AUTO) {

@@ -13,8 +13,8 @@
 //     registers as the MFMA fragments for the whole kernel) and walks the columns of C in tiles of
 //     64: the matching 64 rows of B (K-major) come into LDS by direct-to-LDS buffer loads, double
 //     buffered, and each wavefront multiplies its 32 x 64 block (two 32x32 accumulators of
-//     v_mfma_f32_32x32x2_f32, the tile kernels' depth permutation, so the same sums in the same
-//     order as every tile: bit-identical results) and stores it with non-temporal buffer stores.
+//     v_mfma_f32_32x32x2_f32, the fp32 tiles' depth permutation, so the same sums in the same
+//     order as those tiles': bit-identical results) and stores it with non-temporal buffer stores.
 //   - The loop never waits for its stores: before each tile's barrier a wavefront waits only until
 //     its copy of the next B tile has landed (vmcnt counts in issue order, so that is "all but the
 //     last tile's stores", the immediate kStoresPerTile) and the barrier is a bare s_barrier.

@@ -400,7 +400,7 @@ __device__ __forceinline__ void plain_blocks(floatx16 (&acc)[FM][FN], const floa
 }
 
 // The tile through LDS. Bound at 4096^3 (256x256 tiles, one per CU) by the matrix cores' power:
-// they are busy 64 % of the cycles at 1.7 GHz; 555-607 us by box and clock, 226-247 TFLOP/s of
+// they are busy 71 % of the cycles at 1.84 GHz; 555-607 us by box and clock, 226-247 TFLOP/s of
 // fp32 product, 1.36-1.48 PFLOP/s of bf16, against 961 us on the fp32 matrix cores. Smaller tiles
 // are bound by LDS reads (three planes of each fragment) and by the cuts, 11 vector operations a
 // pair of elements, which a tile of B rows and columns spreads over B products each.

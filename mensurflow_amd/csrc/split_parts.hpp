@@ -44,8 +44,9 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The six part products of fp32 precision, smallest first. Every tile adds them in this order,
-// depth step by depth step, so all tiles give the same bits.
+// The six part products of fp32 precision, smallest first. The tiles through LDS add them in this
+// order, 16-deep step by step, so they give the same bits; the register forms' wavefronts each add
+// every eighth step and their sums are added at the end.
 constexpr int kPartA[6] = {2, 0, 1, 1, 0, 0};
 constexpr int kPartB[6] = {0, 2, 1, 0, 1, 0};
 
