@@ -160,7 +160,10 @@ __device__ __forceinline__ void softmax_step(floatx16 (&s)[SUB], floatx16 (&o)[D
 //     output's own rounding. A smaller output is run again, but one of exactly 0 only where values
 //     under 2^-49 were met: without them it stands for weights below 2^-73, 2^-122 in all.
 // So zero values, and a few tiny ones among others, cost nothing.
-constexpr uint32_t kSmallestValue = (127u - 49u) << 23;
+// Magnitudes are compared as float bits without the sign, times two, minus 1: one operation an
+// element, zero wraps past every other value.
+__device__ __forceinline__ uint32_t magnitude(float v) { return (__float_as_uint(v) << 1) - 1; }
+constexpr uint32_t kSmallestValue = ((127u - 49u) << 24) - 1; // 2^-49
 constexpr float kMostSquares = 0x1p126f;
 
 // The wavefront's queries on the fp32 matrix cores, straight from global memory, scaled after their
@@ -241,10 +244,11 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
     constexpr int kPer = (kUnits + THREADS - 1) / THREADS;
     __shared__ uint4 k_tile0[kPiecesK], k_tile1[kPiecesK];
     __shared__ uint4 v_tile0[kPiecesV], v_tile1[kPiecesV];
-    __shared__ uint32_t smallest;
-    __shared__ float k_squares_of[WAVES], v_squares_of[WAVES];
+    __shared__ uint32_t smallest, large_keys;
+    __shared__ float4 v_squares_of[WAVES / 4];
     if (threadIdx.x == 0) {
         smallest = 0xffffffffu;
+        large_keys = 0;
     }
 
     const BlockWork work = block_work(p);
@@ -296,7 +300,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
     float k_reg[kPer][8], v_reg[kPer][8];
     const float* k_base = p.k + work.off_k;
     const float* v_base = p.v + work.off_v;
-    uint32_t least = 0xffffffffu; // smallest nonzero |v| as bits - 1
+    uint32_t least = 0xffffffffu; // the smallest nonzero value's magnitude
     const auto load = [&](int64_t blk) __attribute__((always_inline)) {
         const int64_t k0 = blk * BK;
 #pragma unroll
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                least = min(least, (__float_as_uint(v_reg[i][j]) & 0x7fffffffu) - 1);
+                least = min(least, magnitude(v_reg[i][j]));
             }
             cut_eight(v_reg[i], part, v_squares);
 #pragma unroll
@@ -466,24 +470,24 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
         }
     }
 
-    if (__any(least < kSmallestValue - 1)) {
+    if (__any(least < kSmallestValue)) {
         atomicMin(&smallest, least);
     }
-    k_squares = mfr::dev::butterfly_sum(k_squares);
+    if (!(k_squares < kMostSquares / THREADS)) {
+        large_keys = 1;
+    }
     v_squares = mfr::dev::butterfly_sum(v_squares);
     if (lane == 0) {
-        k_squares_of[wave] = k_squares;
-        v_squares_of[wave] = v_squares;
+        reinterpret_cast<float*>(v_squares_of)[wave] = v_squares;
     }
     lds_barrier();
     if (!wave_live) {
         return;
     }
-    k_squares = v_squares = 0.0f;
+    v_squares = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-        k_squares += k_squares_of[w];
-        v_squares += v_squares_of[w];
+    for (const float4& four : v_squares_of) {
+        v_squares += (four.x + four.y) + (four.z + four.w);
     }
     float total = sum_halves(run.sum);
     float zero = total * 0.0f; // NaN once a result is not finite
@@ -497,20 +501,19 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
         }
     }
     const float bound =
-        static_cast<float>(k_end) * 0x1p-97f * (8.0f + fminf(sqrtf(v_squares), 0x1p127f));
-    bool again = zero != 0.0f || !(q_squares < kMostSquares) || !(k_squares < kMostSquares);
+        static_cast<float>(k_end) * 0x1p-97f * (8.0f + fminf(__builtin_amdgcn_sqrtf(v_squares), 0x1p127f));
+    bool again = zero != 0.0f || !(q_squares < kMostSquares) || large_keys != 0;
     if (__any(least_out < bound) && !__any(again)) {
-        // The least output that is not 0, as bits - 1 (0 wraps past all), against the bound.
+        // The least output that is not 0.
         uint32_t nonzero = 0xffffffffu;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                nonzero = min(nonzero, (__float_as_uint(oacc[b][e]) & 0x7fffffffu) - 1);
+                nonzero = min(nonzero, magnitude(oacc[b][e]));
             }
         }
-        again = nonzero < __float_as_uint(bound) - 1 ||
-                (least_out == 0.0f && smallest < kSmallestValue - 1);
+        again = nonzero < magnitude(bound) || (least_out == 0.0f && smallest < kSmallestValue);
     }
     if (__any(again)) {
         plain_queries<D, MASK>(p, work, mask_row, wq0, k_end, half, r32, oacc, run);
