@@ -255,9 +255,11 @@ void run_decode(mfr_stream& s, const AttnParams& p, int64_t d) {
             static_cast<size_t>(p.batch_count * p.lq * ranges * (d + 2)) * sizeof(float);
         // Under stream capture one range: a graph would keep the workspace's address, which a later
         // call may free to grow it, and its replays may run beside calls that use it.
+        // (The default stream cannot be asked while another captures: one range then, too.)
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        mfr::check(hipStreamIsCapturing(s.stream, &capture), "hipStreamIsCapturing");
-        if (capture == hipStreamCaptureStatusNone) {
+        if (hipStreamIsCapturing(s.stream, &capture) != hipSuccess) {
+            (void)hipGetLastError();
+        } else if (capture == hipStreamCaptureStatusNone) {
             try {
                 parts = static_cast<float*>(s.reserve(bytes));
             } catch (const mfr::Error&) {
