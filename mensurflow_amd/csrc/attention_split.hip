@@ -156,10 +156,12 @@ __device__ __forceinline__ void softmax_step(floatx16 (&s)[SUB], floatx16 (&o)[D
 //     exponent. With the squares of the workgroup's keys and of the lane's query (both as cut)
 //     summing to less than 2^126, that is under 2^-58;
 //   - an output may have: its terms lose at most 2^-126 (6 + |v|) a key. 2^26 times as much, with a
-//     little room (the bound below, the sum of the squares for the largest value), stays under the
-//     output's own rounding. A smaller output is run again, but one of exactly 0 only where values
-//     under 2^-49 were met: without them it stands for weights below 2^-73, 2^-122 in all.
+//     little room (the bound at the kernel's end, with the root of the sum of all squares for the
+//     largest value), stays under the output's own rounding. A smaller output is run again, but one
+//     of exactly 0 only where values under 2^-49 were met: without them its products are zeros, or
+//     under 2^-126 each, of weights below 2^-77.
 // So zero values, and a few tiny ones among others, cost nothing.
+//
 // Magnitudes are compared as float bits without the sign, times two, minus 1: one operation an
 // element, zero wraps past every other value.
 __device__ __forceinline__ uint32_t magnitude(float v) { return (__float_as_uint(v) << 1) - 1; }
@@ -500,8 +502,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_split_kernel(
             least_out = fminf(least_out, __builtin_fabsf(oacc[b][e]));
         }
     }
-    const float bound =
-        static_cast<float>(k_end) * 0x1p-97f * (8.0f + fminf(__builtin_amdgcn_sqrtf(v_squares), 0x1p127f));
+    const float bound = static_cast<float>(k_end) * 0x1p-97f *
+                        (8.0f + fminf(__builtin_amdgcn_sqrtf(v_squares), 0x1p127f));
     bool again = zero != 0.0f || !(q_squares < kMostSquares) || large_keys != 0;
     if (__any(least_out < bound) && !__any(again)) {
         // The least output that is not 0.

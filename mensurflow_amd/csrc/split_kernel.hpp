@@ -872,7 +872,8 @@ __global__ __launch_bounds__(WAVES_K * 64) void sgemm_split_regs_kernel(GemmPara
         return;
     }
     if (__builtin_amdgcn_readfirstlane(stand == Sums::kNotFinite || under > 0) != 0) {
-        plain_blocks<1, 1, AK, BK>(mine, a_base, b_base, p, kk, w.rows_a, w.rows_b, row0, col0, half, r32);
+        plain_blocks<1, 1, AK, BK>(mine, a_base, b_base, p, kk, w.rows_a, w.rows_b, row0, col0,
+                                   half, r32);
     }
     finish_tile<BM, BN, 32, 32, 1, 1>(mine, p, w, set / FN, set % FN, half, r32, gelu_table);
 }
