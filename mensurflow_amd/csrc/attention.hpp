@@ -58,14 +58,15 @@ __device__ inline BlockWork block_work(const AttnParams& p) {
 // The most queries the decode form takes.
 constexpr int64_t kDecodeMaxQueries = 4;
 
-// Whether the decode form takes 1 to 4 queries against lk keys. It reads K and V once at the HBM's rate and cuts long key counts over the chip, but
-// each query is vector work for every lane, and joining the lane groups costs 5 us at d = 32.
+// Whether the decode form takes 1 to 4 queries against lk keys. It reads K and V once at the HBM's
+// rate and cuts long key counts over the chip, but each query is vector work for every lane, and
+// joining the lane groups of 4 queries costs 4 us at d = 32.
 // Times of the tile kernels over the decode form's (2 to 20000 heads, 4 to 16384 keys):
 //   - 1 query: 0.97 to 26 everywhere;
 //   - 2 queries: 1.0 to 22, but d = 16 below 256 keys 0.45-0.8, d = 32 below 128 keys 0.75-1.0;
 //   - 3 or 4, d a multiple of 32: 1.05 to 8.7 where the heads leave half the chip idle, from 128
-//     keys (d = 32: 256, d = 128: 64) on; with 256 heads or more 0.25-1.0 (20000 x 4 x 16 x 32: 185 us against
-//     668), but d = 32 from 2048 keys on, 1.0 to 1.7;
+//     keys (d = 32: 256, d = 128: 64) on; with 256 heads or more 0.25-1.0 (20000 x 4 x 16 x 32: 185
+//     us against 668), but d = 32 from 2048 keys on, 1.0 to 1.7;
 //   - 3 or 4, d = 16 and 48: 1.2 to 16 for as long key counts as below, 0.15-0.9 under them;
 //     d = 80 and 112: 1.1 to 16 everywhere.
 inline bool decode_takes(int64_t lq, int64_t lk, int64_t d, int64_t batch_count, int cus) {

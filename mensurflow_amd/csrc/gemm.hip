@@ -849,8 +849,9 @@ Plan plan_sgemm(const mfr_gemm_desc& d, int cus) {
     tile_plan(plan);
     // AUTO staging under the 256x256 tile: an operand whose unit stride runs along its rows (M
     // or N) is read in place instead. Its loads are 4 bytes a lane along whole lines either way, so a
-    // copy gains nothing; along the depth the tile loads 16 bytes at any 4-byte alignment, and a copy
-    // saves a cache line in four (4096 x 4096 x 1023 161.6 us in place, 1024 deep 160.4).
+    // copy gains nothing. Along the depth the tile loads 16 bytes at any 4-byte alignment, so a copy
+    // has little to win either (4096 x 4096 x 1023 161.6 us in place, 1024 deep 160.4); the plan's
+    // tests hold it.
     if (d.stage == MFR_STAGE_AUTO && plan.regions[0].tile == MFR_TILE_256x256 &&
         ((plan.stage_a && !plan.ak) || (plan.stage_b && !plan.bk))) {
         Plan partial = plan;
